@@ -28,11 +28,12 @@ FLAGS = [
 ]
 
 
-# Per-source additions.  The scorer keeps MFMA accumulators in VGPRs: its
+# Per-source additions.  The scorers keep MFMA accumulators in VGPRs: their
 # softmax reads every accumulator, and with the compiler's AGPR choice each
 # read is an extra v_accvgpr_read.
 EXTRA_FLAGS = {
     "hc_score.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "hc_colsum.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

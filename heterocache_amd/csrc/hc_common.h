@@ -262,6 +262,21 @@ __device__ __forceinline__ float rows4_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// 16 bytes per lane straight from global memory into LDS: lane i's bytes
+// land at lds + 16*i (lds is wave-uniform).
+__device__ __forceinline__ void lds_dma16(const void* src, void* lds) {
+  __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
+}
+// s_waitcnt vmcnt(0): every LDS-DMA load of this wave has landed.
+__device__ __forceinline__ void wait_lds_dma() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+// s_waitcnt vmcnt(N): all but this wave's N most recent vector loads have
+// landed (loads complete in order).
+template <int N>
+__device__ __forceinline__ void wait_lds_dma_but() {
+  static_assert(N >= 0 && N < 16, "vmcnt field");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | N);
+}
+
 // Order-preserving uint32 key of a float score (larger float, larger key;
 // -0 ranks equal to +0), used by every selection over scores.
 __device__ __forceinline__ uint32_t order_key(float f) {

@@ -131,21 +131,6 @@ __global__ __launch_bounds__(256) void v_tiles_kernel(const PfArgs a) {
   }
 }
 
-// 16 bytes per lane straight from global memory into LDS: lane i's bytes
-// land at lds + 16*i (lds is wave-uniform).
-__device__ __forceinline__ void lds_dma16(const void* src, void* lds) {
-  __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
-}
-// s_waitcnt vmcnt(0): every LDS-DMA load of this wave has landed.
-__device__ __forceinline__ void wait_lds_dma() { __builtin_amdgcn_s_waitcnt(0x0f70); }
-// s_waitcnt vmcnt(N): all but this wave's N most recent vector loads have
-// landed (loads complete in order).
-template <int N>
-__device__ __forceinline__ void wait_lds_dma_but() {
-  static_assert(N >= 0 && N < 16, "vmcnt field");
-  __builtin_amdgcn_s_waitcnt(0x0f70 | N);
-}
-
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_attn_kernel(const PfArgs a) {
   typedef typename Elem<T>::vec8 vec8;

@@ -136,10 +136,6 @@ class H2OKVCluster:
     prompt position pays each key (softmax over all keys, no mask, float32),
     summed over all query positions; the top capacity keys are kept."""
 
-    # Query rows per hc_score call: the scorer holds at most 256 rows of a
-    # 16-bit type, 128 of float32.
-    QUERY_CHUNK = {torch.float32: 128}
-
     def __init__(self, window_size=64, compression_ratio=0.5, kernel_size=5, pooling="avgpool", merge=None):
         self.window_size = window_size
         self.compression_ratio = compression_ratio
@@ -157,31 +153,7 @@ class H2OKVCluster:
 
     def heavy_hitter_scores(self, key_states, query_states):
         """[B*H, L] float32: sum over every query position of its softmax row."""
-        B, H, L, D = query_states.shape
-        scores = torch.empty((B * H, 1, L), dtype=torch.float32, device=query_states.device)
-        k_off = ops.to_device([b * key_states.stride(0) + h * key_states.stride(1) for b in range(B) for h in range(H)],
-                              query_states.device, torch.int64)
-        base = [b * query_states.stride(0) + h * query_states.stride(1) for b in range(B) for h in range(H)]
-        flags = _lib.HC_SCORE_SUM_WINDOW
-        chunk = self.QUERY_CHUNK.get(query_states.dtype, 256)
-        # Row blocks: full chunks, then the tail split into a multiple of 16
-        # and powers of two (the window sizes a summed scorer call takes).
-        blocks, s = [], 0
-        while L - s >= chunk:
-            blocks.append((s, chunk))
-            s += chunk
-        tail = L - s
-        for w in ([tail // 16 * 16] if tail >= 16 else []) + [b for b in (8, 4, 2, 1) if tail % 16 & b]:
-            blocks.append((s, w))
-            s += w
-        # Every block's query offsets in one host-to-device copy.
-        q_offs = ops.to_device(np.asarray([[o + s * query_states.stride(2) for o in base] for s, _ in blocks],
-                                          dtype=np.int64), query_states.device)
-        for i, (s, w) in enumerate(blocks):
-            ops.score(query_states, q_offs[i], query_states.stride(1), query_states.stride(2), key_states, k_off,
-                      key_states.stride(2), L, 1, w, L, "avgpool", 1, 1.0 / math.sqrt(D),
-                      flags=flags | (_lib.HC_SCORE_ACCUMULATE if s else 0), out=scores)
-        return scores.view(B * H, L)
+        return ops.attn_column_sums(query_states, key_states, 1.0 / math.sqrt(query_states.shape[-1]))
 
     def update_kv(self, key_states, query_states, value_states, attention_mask, num_key_value_groups):
         assert key_states.shape[-2] == query_states.shape[-2]

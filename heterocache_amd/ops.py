@@ -602,6 +602,36 @@ def score_given_stats(q, q_off, q_head_stride, q_row_stride, kstore, row_tile_of
     return out
 
 
+def attn_column_sums(q, k, scale, out=None, stream=None):
+    """[B*H, L] float32: per key, the softmax probability it takes from every
+    query position of its head, summed (no mask; hc_attn_column_sums in
+    include/hc.h).  q, k: [B, H, L, 128], the first L keys of k."""
+    lib = _lib.load()
+    _require_cuda(q, k, out)
+    if q.dtype != k.dtype:
+        raise TypeError("q and k must share a dtype")
+    B, H, L, _ = q.shape
+    if out is None:
+        out = torch.empty((B * H, L), dtype=torch.float32, device=q.device)
+    elif out.dtype != torch.float32 or out.numel() < B * H * L or not out.is_contiguous():
+        raise ValueError("out must be a contiguous float32 tensor of [B * H, L]")
+    if q.numel() == 0:
+        return out
+    if k.stride(2) < HEAD_DIM or k.stride(2) % 8:
+        raise ValueError(f"key token stride {k.stride(2)}")
+    # The kernels read rows in 16-byte units: other layouts are copied first.
+    per16 = 16 // q.element_size()
+    q, k = (t if t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(
+        n == 1 or st % per16 == 0 for n, st in zip(t.shape[:3], t.stride())) else
+        t.clone(memory_format=torch.contiguous_format) for t in (q, k))
+    strides = np.array([[st if n > 1 else 0 for n, st in zip(t.shape[:3], t.stride())] for t in (q, k)], dtype=np.int64)
+    code = dtype_code(q.dtype)
+    ws = torch.empty(lib.hc_attn_column_sums_workspace(code, B, H, L), dtype=torch.uint8, device=q.device)
+    _lib.check(lib.hc_attn_column_sums(code, _ptr(q), strides.ctypes.data, _ptr(k), strides.ctypes.data + 24, B, H, L,
+                                       float(scale), _ptr(out), _ptr(ws), ws.numel(), _stream(stream, q)))
+    return out
+
+
 def cake_score(q, q_off, q_head_stride, q_row_stride, k, k_off, k_tok_stride, batch, kv_heads, seq_len, group,
                window, scale, gamma, flags=0, out=None, stats=None, stream=None):
     """CAKE scores [batch * kv_heads, seq_len - window] and the float32 device

@@ -333,6 +333,20 @@ int hc_gather_rows(int dtype, const void* src_k, const void* src_v, const int64_
 int hc_head_pool(int dtype, const void* attn, int64_t batch_stride, int64_t head_stride, int batch, int heads_out,
                  int group, int span, int kernel, float* out, void* stream);
 
+/*
+ * Column sums of a whole prompt's attention, float32, no mask:
+ *   out[(b*heads + h)*seq_len + t] = sum_{i < seq_len} softmax_t(scale * q[b,h,i] . k[b,h,t])
+ * q_strides / k_strides: host arrays of 3 element strides (batch, head,
+ * token; channels contiguous), multiples of 16 bytes, bases 16-byte aligned;
+ * scale finite and positive.  workspace: hc_attn_column_sums_workspace bytes.
+ * Replaces the heavy-hitter sums of H2OKVCluster.update_kv
+ * (heterocache/kv_cluster.py:434-447).
+ */
+int hc_attn_column_sums(int dtype, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                        int batch, int heads, int seq_len, float scale, float* out, void* workspace,
+                        size_t workspace_bytes, void* stream);
+size_t hc_attn_column_sums_workspace(int dtype, int batch, int heads, int seq_len);
+
 /* hc_score flags */
 #define HC_SCORE_CAUSAL_WINDOW 1 /* window row w sees keys t <= L - W + w (kv_cluster.py:169-175) */
 #define HC_SCORE_SUM_WINDOW 2    /* sum probabilities over the W rows of a query head (kv_cluster.py:178) */
