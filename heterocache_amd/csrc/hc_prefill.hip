@@ -27,12 +27,17 @@
 //    base-2 softmax per query column, O^T += V^T P^T with P taken straight
 //    from the S accumulators (the tile layout's V token order is the order in
 //    which the accumulator holds the scores), fp32 accumulation;
-//  * the softmax is VALU work beside the MFMAs (CDNA4 issues a wave64 VALU
-//    op over 4 cycles, v_exp at a quarter of that rate), so it is kept lean:
-//    the tile maximum is taken on raw scores and the scale folded into the
-//    exp2 argument's fma, masking runs only on tiles that cross the
-//    diagonal, and O is rescaled only when the running maximum grows by more
-//    than 2^8.
+//  * the softmax is VALU work beside the MFMAs (a SIMD's 16 MFMAs alone take
+//    131 ns, with the exponentials and fmas of their softmax among them up to
+//    190), so it is kept lean: the scale is folded into the exp2 argument's
+//    fma, masking runs only on tiles that cross the diagonal, and no maximum
+//    is taken in the loop -- the running reference moves, and O is rescaled,
+//    only when a tile's probability sums, which are formed anyway, exceed
+//    kPfLazy.  Without the 32 maxima a lane and their cross-lane folds per 64
+//    keys: 15.41 -> 14.66 ms for 8192 queries over 131072 keys (32 heads over
+//    8, bf16; 1105 -> 1162 TFLOP/s), 0.53 -> 0.50 ms for 8003 over 8003.
+//    (48 or 64 queries a wave, so that an LDS read feeds 3 or 4 MFMAs, leave
+//    two waves or one per SIMD: 15.9 and 19.5 ms.)
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -50,7 +55,7 @@ constexpr int kPfBlockQ = kPfWaves * kPfWaveQ;  // queries per workgroup
 constexpr int kPfTiles = 2;                     // 32-token tiles per iteration
 constexpr int kPfKeys = kPfTiles * HC_TILE;     // keys per iteration
 constexpr int kPfThreads = kPfWaves * 64;
-constexpr float kPfLazy = 8.f;                  // lazy-rescale threshold, log2 units
+constexpr float kPfLazy = 256.f;                // lazy-rescale threshold: a lane's sum of probabilities of a tile
 
 struct PfArgs {
   const void* q;
@@ -304,20 +309,36 @@ __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_at
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        // Raw tile maximum (scale > 0), shared by the 4 lanes of a query.
-        float mx = -INFINITY;
+        // Probabilities against the reference maximum m, their sum and their
+        // packed form.
+        float ps;
+        auto probs = [&](float nm) {
+          ps = 0.f;
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb)
+          for (int c = 0; c < 2; ++c) {
+            float pv[8];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sacc[tb][j][r]);
-        mx = rows4_max(mx);
-        const float mt = mx * a.scale_log2;
-        // Lazy rescaling: the reference maximum m only moves when a tile
-        // maximum exceeds it by more than kPfLazy (log2 units), so the O
-        // rescale runs on a few tiles per row; probabilities stay below
-        // 2^kPfLazy, well inside every input type's range.
-        if (__any(mt > m[j] + kPfLazy)) {
-          const float mnew = fmaxf(m[j], mt);
+            for (int e = 0; e < 8; ++e) {
+              pv[e] = fast_exp2(fmaf(sacc[2 * c + (e >> 2)][j][e & 3], a.scale_log2, nm));
+              ps += pv[e];
+            }
+            pb[c][j] = pack8<T>(pv);
+          }
+        };
+        probs(-m[j]);
+        // m only moves when a lane's sum of the tile exceeds kPfLazy (or is
+        // NaN, as in a row's first tile, where m = -inf): the sums are formed
+        // anyway, so the maxima, their fold over the 4 lanes of a query and
+        // the O rescale run on a few tiles per row.  Probabilities stay below
+        // kPfLazy, well inside every input type's range.
+        if (__any(!(ps <= kPfLazy))) {
+          // Raw tile maximum (scale > 0), shared by the 4 lanes of a query.
+          float mx = -INFINITY;
+#pragma unroll
+          for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sacc[tb][j][r]);
+          const float mnew = fmaxf(m[j], rows4_max(mx) * a.scale_log2);
           const float alpha = m[j] == -INFINITY ? 0.f : fast_exp2(m[j] - mnew);
           m[j] = mnew;
           l[j] *= alpha;
@@ -325,24 +346,9 @@ __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_at
           for (int db = 0; db < 8; ++db)
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[db][j][r] *= alpha;
+          probs(mnew == -INFINITY ? 0.f : -mnew);
         }
-        const float nm = -m[j];
-        float p[4][4];
-        float ps = 0.f;
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[tb][r] = fast_exp2(fmaf(sacc[tb][j][r], a.scale_log2, nm));
-            ps += p[tb][r];
-          }
         l[j] += ps;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const float pv[8] = {p[2 * c][0],     p[2 * c][1],     p[2 * c][2],     p[2 * c][3],
-                               p[2 * c + 1][0], p[2 * c + 1][1], p[2 * c + 1][2], p[2 * c + 1][3]};
-          pb[c][j] = pack8<T>(pv);
-        }
       }
       __builtin_amdgcn_s_setprio(0);
     }
@@ -395,8 +401,8 @@ __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_at
     const float inv = 1.f / lt;
     // The softmax state of query qi over its visible keys: m is a reference
     // point of the scaled base-2 scores, not a bound -- the lazy rescale
-    // lets the true maximum sit up to kPfLazy above it, so a single
-    // exp2(score - m) can reach 2^kPfLazy -- and lt is the sum of
+    // lets the true maximum sit up to log2(kPfLazy) above it, so a single
+    // exp2(score - m) can reach kPfLazy -- and lt is the sum of
     // exp2(score - m).  Consumers use only m + log2(lt), the log-sum-exp,
     // which is exact whatever m is; one that needs p <= 1 per term must
     // renormalise first.
@@ -437,6 +443,7 @@ __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_at
 constexpr int kDvPitch = HC_TILE + 8;            // fp32: transposed V row, 32 k-slots + skew
 constexpr int kDvNPitch = HC_HEAD_DIM + 16;      // 16-bit: natural V row, 128 channels + skew
 constexpr int kDvWaves = 4;
+constexpr float kDvLazy = 8.f;                   // lazy-rescale threshold, log2 units
 
 // Per-wave V buffer (elements): fp32 keeps the tile transposed ([channel][k-slot]);
 // 16-bit types keep it in natural layout ([token][channel]) and read the A
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
       for (int j = 0; j < 4; ++j) mx = fmaxf(mx, sacc[h][j]);
     mx = rows4_max(mx);
     const float mt = mx * a.scale_log2;
-    if (__any(mt > m + kPfLazy)) {
+    if (__any(mt > m + kDvLazy)) {
       const float mnew = fmaxf(m, mt);
       const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mnew);
       m = mnew;

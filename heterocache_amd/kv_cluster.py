@@ -25,7 +25,7 @@ import math
 import numpy as np
 import torch
 
-from . import _lib, compress, ops
+from . import compress, ops
 
 
 def _round_dtype(dtype, round_scores):

@@ -76,6 +76,23 @@ def test_prefill_matches_oracle(dev, dt, case):
     assert err <= ATTN_TOL[dt], f"max-abs {err}"
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("case", [(1, 2, 1, 200, 640), (1, 2, 1, 60, 1500)])  # one pass; keys split
+def test_prefill_growing_maxima(dev, dt, case):
+    """Keys whose logits grow along the prompt, so that the softmax reference
+    moves in many tiles, and a key that dominates after thousands of others."""
+    B, Hq, Hkv, Lq, Lk = case
+    print(f"prefill growing maxima dt={dt} {case}", flush=True)
+    q, k, v = _inputs(dev, dt, B, Hq, Hkv, Lq, Lk, 77, pad=40)
+    k.mul_(0.1).add_((torch.linspace(0.0, 3.0, Lk, device=dev)[:, None] * q[0, 0, 5].float() / 12).to(k.dtype))
+    k[:, :, Lk - Lq // 2] = 4 * q[:, :1, 9]
+    scale = 1.0 / math.sqrt(128)
+    got = as_np(ops.prefill_attn(q, k, v, scale))
+    ref = O.prefill_attention(as_np(q), as_np(k), as_np(v), scale)
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() <= ATTN_TOL[dt]
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
 def test_prefill_projection_layout_and_out_view(dev, dt):
     """Inputs as transposed [B, L, H, 128] views; output written into a view
