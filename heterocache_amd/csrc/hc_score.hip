@@ -19,16 +19,19 @@
 //     the A operand, loaded straight from HBM; queries are B operands staged
 //     in LDS once per workgroup), reduced to a (max, sum exp) per row; with
 //     fewer than 32 rows the logits are stored too.
+//     Under the cast chain the stored logits are 16-bit (see Logit), and
+//     summed windows of up to kCastLogitRows rows store them too.
 //  2. score_stats_merge_kernel: fold the workgroups' (max, sum) per row
 //     (on the stored-logit path, phase 3b folds them itself unless the
 //     drift histograms need clearing).
-//  3a. (>= 32 rows) score_probs_kernel: recompute the logits, normalise, sum
+//  3a. (>= 32 rows, no stored logits) score_probs_kernel: recompute the logits, normalise, sum
 //     over the window rows of each query head (xor-shuffle tree: fixed
 //     order), write A[job][w'][g][t]; score_pool_kernel: pooling over t and
 //     max over g -> S[job][w'][t].
-//  3b. (< 32 rows) score_finish_kernel: the same from the stored logits
-//     (score_finish_reg_kernel for pool kernels 5 and 7: pooling in
-//     registers).
+//  3b. (stored logits) score_finish_kernel: the same from the stored logits
+//     (for pool kernels 5 and 7 score_finish_reg_kernel: pooling in
+//     registers; under the cast chain score_finish_cast_kernel and
+//     score_finish_window_kernel).
 // CAKE scoring (hc_cake_score) runs phases 1-2, the probability pass with
 // window moments, and its own pooling and reductions.
 // With the rows' softmax statistics already known (prefill attention reports
@@ -148,10 +151,61 @@ __device__ __forceinline__ float scaled_logit(const ScoreArgs& a, float acc) {
   return round_fixed<RM>(round_fixed<RM>(acc) * a.scale) * 1.4426950408889634f;
 }
 
+// Stored logits.  Without casts the base-2 logits, float32, rows of `span`.
+// Under the cast chain a logit is a value of the model's 16-bit type before
+// its factor log2(e), so that value is stored in that type (exactly; half the
+// traffic) and the factor is applied, in float32 as ever, where it is read;
+// rows are padded to whole 16-byte units.
+template <int RM>
+struct Logit {
+  typedef float type;
+  static constexpr int kUnit = 1;
+};
+template <>
+struct Logit<1> {
+  typedef __bf16 type;
+  static constexpr int kUnit = 8;
+};
+template <>
+struct Logit<2> {
+  typedef _Float16 type;
+  static constexpr int kUnit = 8;
+};
+__host__ __device__ inline int64_t cast_logit_pitch(int span) { return ((int64_t)span + 7) / 8 * 8; }
+template <int RM>
+__device__ __forceinline__ typename Logit<RM>::type* logit_row(void* logits, int64_t row, int span) {
+  return reinterpret_cast<typename Logit<RM>::type*>(logits) + row * (RM == 0 ? span : cast_logit_pitch(span));
+}
+template <int RM>
+__device__ __forceinline__ const typename Logit<RM>::type* logit_row(const void* logits, int64_t row, int span) {
+  return logit_row<RM>(const_cast<void*>(logits), row, span);
+}
+// The stored form of a dot product, and the base-2 logit of a stored value.
+template <int RM>
+__device__ __forceinline__ float stored_logit(const ScoreArgs& a, float acc) {
+  if constexpr (RM == 0) return acc * a.scale2;
+  return round_fixed<RM>(round_fixed<RM>(acc) * a.scale);
+}
+template <int RM>
+__device__ __forceinline__ float base2_logit(float stored) {
+  return RM == 0 ? stored : stored * 1.4426950408889634f;
+}
+template <int RM>
+__device__ __forceinline__ f32x4 read_logits4(const typename Logit<RM>::type* p) {
+  if constexpr (RM == 0) {
+    return *reinterpret_cast<const f32x4*>(p);
+  } else {
+    typedef typename Logit<RM>::type v4 __attribute__((ext_vector_type(4)));
+    const v4 x = *reinterpret_cast<const v4*>(p);
+    return f32x4{base2_logit<RM>((float)x[0]), base2_logit<RM>((float)x[1]), base2_logit<RM>((float)x[2]),
+                 base2_logit<RM>((float)x[3])};
+  }
+}
+
 // Logits (base 2) of row 16nt + (lane & 15) (visible up to `limit`) for
 // tokens t0 + 4*(lane>>4) + j; keys are the A operand.  RAW (no casts):
 // the unscaled dot products, the caller folds scale2 into its exp2 argument.
-template <typename T, int RM, bool MASK, bool RAW = false>
+template <typename T, int RM, bool MASK, bool RAW = false, bool STORED = false>
 __device__ __forceinline__ void subtile_logits(const ScoreArgs& a, const typename Elem<T>::vec8 (&kr)[4],
                                                const T* s_q, int nt, int t0, int lane, int limit, float (&x)[4]) {
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -161,7 +215,8 @@ __device__ __forceinline__ void subtile_logits(const ScoreArgs& a, const typenam
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int t = t0 + 4 * (lane >> 4) + j;
-    x[j] = (!MASK || t <= limit) ? (RAW ? acc[j] : scaled_logit<RM>(a, acc[j])) : -INFINITY;
+    x[j] = (!MASK || t <= limit) ? (RAW ? acc[j] : STORED ? stored_logit<RM>(a, acc[j]) : scaled_logit<RM>(a, acc[j]))
+                                 : -INFINITY;
   }
 }
 
@@ -191,8 +246,8 @@ __device__ __forceinline__ void load_k_chunk(const ScoreArgs& a, const T* kj, in
 // variants the kernel outgrows the instruction cache.
 template <typename T, int RM, bool LOGITS, bool MASK>
 __device__ __forceinline__ void stats_chunk(const ScoreArgs& a, const KRegs<T>& k, const T* s_q, float* my, int job,
-                                            int tw, int lane, float* __restrict__ logits) {
-  const bool vec_logits = (a.span & 3) == 0;
+                                            int tw, int lane, void* __restrict__ logits) {
+  const bool vec_logits = RM != 0 || (a.span & 3) == 0;
   for (int nt = 0; nt < a.NT; ++nt) {
     const int limit = row_limit(a, 16 * nt + (lane & 15));
     // All sub-tiles' logits first (independent MFMA chains, no branch
@@ -203,20 +258,24 @@ __device__ __forceinline__ void stats_chunk(const ScoreArgs& a, const KRegs<T>& 
     float x[kSubTiles][4];
 #pragma unroll
     for (int u = 0; u < kSubTiles; ++u) {
-      subtile_logits<T, RM, MASK, RAW>(a, k.v[u], s_q, nt, tw + 16 * u, lane, limit, x[u]);
+      subtile_logits<T, RM, MASK, RAW, LOGITS>(a, k.v[u], s_q, nt, tw + 16 * u, lane, limit, x[u]);
       if constexpr (LOGITS) {
-        // Row r, tokens t..t+3 (16 bytes) of the job's [R][span] logits.
+        // Row r, tokens t..t+3 (one vector) of the job's [R][span] logits.
+        typedef typename Logit<RM>::type LT;
         const int r = 16 * nt + (lane & 15), t = tw + 16 * u + 4 * (lane >> 4);
-        float* o = logits + ((int64_t)job * a.R + r) * a.span + t;
+        LT* o = logit_row<RM>(logits, (int64_t)job * a.R + r, a.span) + t;
         if (r < a.R) {
-          if (vec_logits && t + 4 <= a.span) {
-            *reinterpret_cast<f32x4*>(o) = f32x4{x[u][0], x[u][1], x[u][2], x[u][3]};
+          if (vec_logits && (RM != 0 ? t < a.span : t + 4 <= a.span)) {
+            typedef LT v4 __attribute__((ext_vector_type(4)));
+            *reinterpret_cast<v4*>(o) = v4{(LT)x[u][0], (LT)x[u][1], (LT)x[u][2], (LT)x[u][3]};
           } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-              if (t + j < a.span) o[j] = x[u][j];
+              if (t + j < a.span) o[j] = (LT)x[u][j];
           }
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[u][j] = base2_logit<RM>(x[u][j]);
       }
     }
     // -FLT_MAX (not -inf) as the empty maximum: exp2(-inf - m) = 0 for a
@@ -259,7 +318,7 @@ __device__ __forceinline__ void stats_chunk(const ScoreArgs& a, const KRegs<T>& 
 // and was slower: the passes are bound by latency within a chunk.)
 template <typename T, bool STORE, int RM, bool LOGITS>
 __global__ __launch_bounds__(kScoreWaves * 64) void score_stats_kernel(ScoreArgs a, float* __restrict__ part,
-                                                                      float* __restrict__ logits) {
+                                                                      void* __restrict__ logits) {
   extern __shared__ __align__(16) unsigned char smem[];
   T* s_q = reinterpret_cast<T*>(smem);
   float* s_st = reinterpret_cast<float*>(smem + (size_t)a.NT * 16 * kQPitch * sizeof(T));  // [waves][rows][2]
@@ -312,8 +371,10 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_stats_kernel(ScoreArgs
 // per 256-byte key row, so the pass is bound by streaming the keys -- and
 // the MFMA operand layout of score_stats_kernel makes every wave load touch
 // 16 rows of 64 bytes each.  Here the 16 lanes of group s hold channels
-// 8c..8c+7 (c = lane % 16) of token 4*step + s, so a wave load reads four
-// whole 256-byte token rows; the groups' partial dot products of all NR
+// 8c..8c+7 (c = lane % 16) of token 8*s + step, so a wave load reads four
+// whole 256-byte token rows, and a lane ends with eight consecutive tokens'
+// logits, stored as whole 16-byte units (eight
+// heads x 128K, four rows: 58.3 -> 53.9 us against scattered float32 stores); the groups' partial dot products of all NR
 // rows are summed by one DPP reduce-scatter (row16_sum_scatter), after which
 // lane c < R of a group holds row c's logit of its token.  Logits are stored as score_stats_kernel stores them (base-2
 // scaled and masked, [job][R][span]) and every workgroup writes one
@@ -352,7 +413,7 @@ __device__ __forceinline__ typename Dot2<T>::pair pair_at(const typename Elem<T>
 
 template <typename T, int NR, int RM>
 __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(ScoreArgs a, float* __restrict__ part,
-                                                                          float* __restrict__ logits) {
+                                                                          void* __restrict__ logits) {
   typedef typename Elem<T>::vec8 vec8;
   __shared__ float s_st[kScoreWaves][16][2];
   const int job = blockIdx.y;
@@ -385,7 +446,8 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(Score
   const int c0 = blockIdx.x * a.cpw, c1 = min(c0 + a.cpw, nchunks);
   const int t_end = min(c1 * kScoreChunk, a.L);
   const T* kb = reinterpret_cast<const T*>(a.k) + a.k_off[job] + 8 * c;
-  float* lrow = logits + ((int64_t)job * a.R + (owner ? c : 0)) * a.span;
+  typedef typename Logit<RM>::type LT;
+  LT* lrow = logit_row<RM>(logits, (int64_t)job * a.R + (owner ? c : 0), a.span);
   float m = -FLT_MAX, l = 0.f;
   constexpr int kIter = kScoreWaves * kRowsSteps * 4;  // tokens per workgroup iteration
   // Keys of one iteration, streamed past L2 (this pass reads them once):
@@ -399,7 +461,7 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(Score
   auto load_keys = [&](vec8 (&kr)[kRowsSteps], int t0) {
 #pragma unroll
     for (int st = 0; st < kRowsSteps; ++st)
-      kr[st] = load8_stream<T>(kb + (int64_t)min(t0 + 4 * st + sub, a.L - 1) * a.k_tok_stride);
+      kr[st] = load8_stream<T>(kb + (int64_t)min(t0 + kRowsSteps * sub + st, a.L - 1) * a.k_tok_stride);
   };
   auto consume = [&](const vec8 (&kr)[kRowsSteps], int t0) {
     float x[kRowsSteps];
@@ -419,18 +481,33 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(Score
         acc[r] = d;
       }
       const float mine = row16_sum_scatter<NR>(acc, lane);  // row c % NR
-      const int t = t0 + 4 * st + sub;
-      x[st] = t <= limit ? scaled_logit<RM>(a, mine) : -INFINITY;
+      const int t = t0 + kRowsSteps * sub + st;
+      x[st] = t <= limit ? stored_logit<RM>(a, mine) : -INFINITY;
     }
     // The logits are stored after all the iteration's keys are consumed:
     // stores between the key waits count against the same in-order counter,
     // so each wait also waited for the next key (prefill compression 0.192-
     // 0.193 -> 0.191 ms per 128K layer).
+    const int tl = t0 + kRowsSteps * sub;
+    if (owner && tl < a.span) {
+      if (RM != 0 || ((a.span & 3) == 0 && tl + kRowsSteps <= a.span)) {
+        typedef LT __attribute__((ext_vector_type(16 / sizeof(LT)))) lvec;
+        constexpr int kLanes = 16 / sizeof(LT);
 #pragma unroll
-    for (int st = 0; st < kRowsSteps; ++st) {
-      const int t = t0 + 4 * st + sub;
-      if (owner && t < a.span) lrow[t] = x[st];
+        for (int v = 0; v < kRowsSteps / kLanes; ++v) {
+          lvec y;
+#pragma unroll
+          for (int e = 0; e < kLanes; ++e) y[e] = (LT)x[v * kLanes + e];
+          *reinterpret_cast<lvec*>(lrow + tl + v * kLanes) = y;
+        }
+      } else {
+#pragma unroll
+        for (int st = 0; st < kRowsSteps; ++st)
+          if (tl + st < a.span) lrow[tl + st] = (LT)x[st];
+      }
     }
+#pragma unroll
+    for (int st = 0; st < kRowsSteps; ++st) x[st] = base2_logit<RM>(x[st]);
     float mx = x[0];
 #pragma unroll
     for (int st = 1; st < kRowsSteps; ++st) mx = __builtin_elementwise_maximum(mx, x[st]);
@@ -1072,7 +1149,7 @@ __device__ __forceinline__ void finish_row_stats(const float* __restrict__ stats
 }
 
 template <int RMODE, int POOL, bool HIST>
-__global__ __launch_bounds__(256) void score_finish_kernel(const float* __restrict__ logits,
+__global__ __launch_bounds__(256) void score_finish_kernel(const void* __restrict__ logits,
                                                            const float* __restrict__ stats,
                                                            const float* __restrict__ part, int nparts, int R, int G, int W,
                                                            int span, int sum_w, int kernel, int accumulate,
@@ -1121,16 +1198,16 @@ __global__ __launch_bounds__(256) void score_finish_kernel(const float* __restri
           f32x4 acc = {0.f, 0.f, 0.f, 0.f};
           for (int w = w_lo; w < w_hi; ++w) {
             const int r = g * W + w;
-            const float* row = logits + ((int64_t)job * R + r) * span;
+            const auto* row = logit_row<RMODE>(logits, (int64_t)job * R + r, span);
             const float m = s_m[r], iz = s_iz[r];
             if (vec_ok) {
-              const f32x4 x = *reinterpret_cast<const f32x4*>(row + tb);
+              const f32x4 x = read_logits4<RMODE>(row + tb);
 #pragma unroll
               for (int e = 0; e < 4; ++e) acc[e] += fin_prob<RMODE>(x[e], m, iz);
             } else {
 #pragma unroll
               for (int e = 0; e < 4; ++e)
-                if (tb + e < span) acc[e] += fin_prob<RMODE>(row[tb + e], m, iz);
+                if (tb + e < span) acc[e] += fin_prob<RMODE>(base2_logit<RMODE>((float)row[tb + e]), m, iz);
             }
           }
 #pragma unroll
@@ -1140,7 +1217,8 @@ __global__ __launch_bounds__(256) void score_finish_kernel(const float* __restri
           float acc = 0.f;
           for (int w = w_lo; w < w_hi; ++w) {
             const int r = g * W + w;
-            acc += fin_prob<RMODE>(logits[((int64_t)job * R + r) * span + th], s_m[r], s_iz[r]);
+            acc += fin_prob<RMODE>(base2_logit<RMODE>((float)logit_row<RMODE>(logits, (int64_t)job * R + r, span)[th]),
+                                   s_m[r], s_iz[r]);
           }
           ah[gg] = round_fixed<RMODE>(acc);
         }
@@ -1207,7 +1285,7 @@ constexpr int kFinRegPos = 8;
 constexpr int kFinRegTile = 256 * kFinRegPos;
 constexpr int kFinRegHistTiles = 2;
 template <int RMODE, int POOL, bool HIST, int P>
-__global__ __launch_bounds__(256) void score_finish_reg_kernel(const float* __restrict__ logits,
+__global__ __launch_bounds__(256) void score_finish_reg_kernel(const void* __restrict__ logits,
                                                                const float* __restrict__ stats,
                                                                const float* __restrict__ part, int nparts, int R,
                                                                int G, int W,
@@ -1260,12 +1338,12 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const float* __re
           for (int i = 0; i < kFinRegPos; ++i) acc[i] = 0.f;
           for (int w = w_lo; w < w_hi; ++w) {
             const int r = g * W + w;
-            const float* row = logits + ((int64_t)job * R + r) * span;
+            const auto* row = logit_row<RMODE>(logits, (int64_t)job * R + r, span);
             const float m = s_m[r], iz = s_iz[r];
             if (vec_ok) {
               f32x4 x[NV];
 #pragma unroll
-              for (int v = 0; v < NV; ++v) x[v] = *reinterpret_cast<const f32x4*>(row + tb + 4 * v);
+              for (int v = 0; v < NV; ++v) x[v] = read_logits4<RMODE>(row + tb + 4 * v);
 #pragma unroll
               for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -1273,7 +1351,7 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const float* __re
             } else {
 #pragma unroll
               for (int i = 0; i < kFinRegPos; ++i)
-                if (tb + i < span) acc[i] += fin_prob_reg<RMODE>(row[tb + i], m, iz);
+                if (tb + i < span) acc[i] += fin_prob_reg<RMODE>(base2_logit<RMODE>((float)row[tb + i]), m, iz);
             }
           }
 #pragma unroll
@@ -1283,7 +1361,8 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const float* __re
           float acc = 0.f;
           for (int w = w_lo; w < w_hi; ++w) {
             const int r = g * W + w;
-            acc += fin_prob_reg<RMODE>(logits[((int64_t)job * R + r) * span + th], s_m[r], s_iz[r]);
+            acc += fin_prob_reg<RMODE>(
+                base2_logit<RMODE>((float)logit_row<RMODE>(logits, (int64_t)job * R + r, span)[th]), s_m[r], s_iz[r]);
           }
           ah[gg] = round_fixed<RMODE>(acc);
         }
@@ -1357,6 +1436,240 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const float* __re
     uint32_t* h = hist + ((int64_t)job * wout + wo) * kKeyDigitBins;
     for (int b = threadIdx.x; b < kKeyDigitBins; b += 256)
       if (s_hist[b]) atomicAdd(&h[b], s_hist[b]);
+  }
+}
+
+// Finish pass under the cast chain (16-bit stored logits, pool kernels 5 and
+// 7, no histogram).  A tile is 512 positions loaded, 16 bytes a lane, of which
+// the middle 496 are pooled: the neighbours are part of the tile, so there is
+// no halo path, and its stride keeps every load aligned.
+// One wave per query head (kFcHeads heads of a group at a time, the next
+// heads' first row in flight meanwhile).  With 2048-position tiles a layer of
+// a 12K prompt (28 heads over 4, float16) had 24 workgroups and took 19.4 us,
+// now 100 and 6.9; 32 heads over 8 x 131072 take 10.6 us as before, with half
+// the logits' bytes.
+constexpr int kFcLoad = 512, kFcOut = kFcLoad - 16;
+constexpr int kFcHeads = 4;
+constexpr int kFcGrid = 1024;
+template <int RM>
+__device__ __forceinline__ void read_logits8(const typename Logit<RM>::type* p, float (&x)[8]) {
+  typedef typename Logit<RM>::type v8 __attribute__((ext_vector_type(8)));
+  const v8 y = *reinterpret_cast<const v8*>(p);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = base2_logit<RM>((float)y[e]);
+}
+// Pooled value around strip position i (P <= 8 neighbours on either side).
+template <int POOL, int P>
+__device__ __forceinline__ float fc_pool(const float* strip, int i) {
+  float v = POOL == 0 ? 0.f : -INFINITY;
+#pragma unroll
+  for (int d = -P; d <= P; ++d) v = POOL == 0 ? v + strip[i + d] : fmaxf(v, strip[i + d]);
+  return v;
+}
+
+template <int RM, int POOL, int P>
+__global__ __launch_bounds__(256) void score_finish_cast_kernel(const void* __restrict__ logits,
+                                                                const float* __restrict__ stats,
+                                                                const float* __restrict__ part, int nparts, int R,
+                                                                int G, int W, int span, int sum_w, int accumulate,
+                                                                float* __restrict__ S) {
+  static_assert(RM != 0 && P <= 8, "16-bit logits, neighbours inside the tile's margin");
+  __shared__ __align__(16) float s_a[2][kFcHeads][kFcLoad];
+  __shared__ float s_m[kLogitRowsMax], s_iz[kLogitRowsMax];
+  const int wout = sum_w ? 1 : W;
+  const int job = blockIdx.y / wout, wo = blockIdx.y % wout;
+  const int w_lo = sum_w ? 0 : wo, w_hi = sum_w ? W : wo + 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ntiles = (span + kFcOut - 1) / kFcOut;
+  constexpr float pad = POOL == 0 ? 0.f : -INFINITY;
+  // This lane's eight positions, tile * kFcOut - 8 + 8 * lane on, of one row.
+  auto row8 = [&](int tile, int g, int w, float (&x)[8]) {
+    const int t = tile * kFcOut - 8 + 8 * lane;
+    if (tile < ntiles && g < G && t >= 0 && t < span) {
+      read_logits8<RM>(logit_row<RM>(logits, (int64_t)job * R + g * W + w, span) + t, x);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = -INFINITY;
+    }
+  };
+  float x[8];
+  row8(blockIdx.x, wave, w_lo, x);  // in flight over the statistics
+  finish_row_stats<false>(stats, part, nparts, job, R, s_m, s_iz);
+  __syncthreads();
+  const float inv_k = 1.f / (float)(2 * P + 1);
+  float* o = S + ((int64_t)job * wout + wo) * span;
+  int buf = 0;
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int o0 = tile * kFcOut;  // first pooled position
+    const int t = o0 - 8 + 8 * lane;
+    float best[2] = {-INFINITY, -INFINITY};
+    for (int g0 = 0; g0 < G; g0 += kFcHeads) {
+      const int g = g0 + wave;
+      if (g < G) {
+        float acc[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+        for (int w = w_lo; w < w_hi; ++w) {
+          const int r = g * W + w;
+          if (w > w_lo) row8(tile, g, w, x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += fin_prob<RM>(x[e], s_m[r], s_iz[r]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = t + e >= 0 && t + e < span ? round_fixed<RM>(acc[e]) : pad;
+        f32x4* d = reinterpret_cast<f32x4*>(&s_a[buf][wave][8 * lane]);
+        d[0] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+        d[1] = f32x4{acc[4], acc[5], acc[6], acc[7]};
+      }
+      if (g0 + kFcHeads < G)
+        row8(tile, g + kFcHeads, w_lo, x);
+      else
+        row8(tile + gridDim.x, wave, w_lo, x);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int i = (int)threadIdx.x + 256 * q;
+        if (i >= kFcOut) continue;
+        for (int gg = 0; gg < kFcHeads && g0 + gg < G; ++gg) {
+          float v = fc_pool<POOL, P>(s_a[buf][gg], 8 + i);
+          if constexpr (POOL == 0) v *= inv_k;
+          best[q] = fmaxf(best[q], round_fixed<RM>(v));
+        }
+      }
+      buf ^= 1;  // the next strips: this buffer may still be read
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = (int)threadIdx.x + 256 * q;
+      if (i < kFcOut && o0 + i < span) o[o0 + i] = accumulate ? o[o0 + i] + best[q] : best[q];
+    }
+  }
+}
+
+// The same for summed windows of whole 16-row tiles (R <= kCastLogitRows):
+// wave rg sums rows 16n + 4rg + [0, 4) of a head's window, and the four
+// waves' sums are added in score_probs_pool_kernel's order, so the scores are
+// the ones that pass forms.  Its second read of the keys (256 bytes a token
+// and job) and their products are replaced by the logits' write and read
+// (2R bytes each).
+// Measured, per call, against two passes over the keys (us): 32 rows, 32 jobs
+// x 8192 keys 39.7 -> 26.6, x 700 18.0 -> 16.6, x 32768 99 -> 86, x 65536 206
+// -> 161; 64 rows, 32 jobs x 8192 50 -> 39, x 16384 (64 MiB of logits) 70 ->
+// 66, 28 jobs x 32768 104 -> 111, 8 jobs x 131072 111 -> 125: the keys still
+// come from the Infinity Cache the second time, and 64 rows of logits are
+// written and read at half their bytes each, so above 32 rows the line lies at
+// kCastLogitBytes.
+constexpr int kCastLogitRows = 64;
+constexpr int64_t kCastLogitBytes = (int64_t)64 << 20;
+template <int RM, int POOL, int P>
+__global__ __launch_bounds__(256) void score_finish_window_kernel(const void* __restrict__ logits,
+                                                                  const float* __restrict__ stats,
+                                                                  const float* __restrict__ part, int nparts, int R,
+                                                                  int G, int W, int span, int accumulate,
+                                                                  float* __restrict__ S) {
+  static_assert(RM != 0 && P <= 8, "16-bit logits, neighbours inside the tile's margin");
+  __shared__ __align__(16) float s_a[4][kFcLoad];
+  __shared__ float s_sum[kFcLoad];
+  __shared__ float s_m[kCastLogitRows], s_iz[kCastLogitRows];
+  __shared__ float s_fold[256][2];
+  const int job = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int o0 = (int)blockIdx.x * kFcOut;
+  const int t = o0 - 8 + 8 * lane;
+  const bool live = t >= 0 && t < span;
+  constexpr float pad = POOL == 0 ? 0.f : -INFINITY;
+  typedef typename Logit<RM>::type v8 __attribute__((ext_vector_type(8)));
+  // Rows 16n + 4 wave + [0, 4) of head g.
+  auto rows4 = [&](int g, int n, v8 (&x)[4]) {
+    const auto* p = logit_row<RM>(logits, (int64_t)job * R + g * W + 16 * n + 4 * wave, span) + (live ? t : 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const v8*>(p + j * cast_logit_pitch(span));
+  };
+  v8 xa[4], xb[4];
+  rows4(0, 0, xa);  // in flight over the statistics
+  if (W > 16) rows4(0, 1, xb);
+  // Row statistics: thread (sub, r) folds parts sub, sub + nsub, ... of row r.
+  const int nsub = 256 / R;
+  {
+    const int r = threadIdx.x % R, sub = threadIdx.x / R;
+    float m = -INFINITY, l = 0.f;
+    if (part) {
+      if (sub < nsub) {
+        const float2* q = reinterpret_cast<const float2*>(part) + (int64_t)job * nparts * R + r;
+#pragma unroll 4
+        for (int c = sub; c < nparts; c += nsub) {
+          const float2 y = q[(int64_t)c * R];
+          merge_ml(m, l, y.x, y.y);
+        }
+      }
+    } else if (sub == 0) {
+      m = stats[((int64_t)job * R + r) * 2];
+      l = stats[((int64_t)job * R + r) * 2 + 1];
+    }
+    s_fold[threadIdx.x][0] = m;
+    s_fold[threadIdx.x][1] = l;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < R) {
+    float m = -INFINITY, l = 0.f;
+    for (int sub = 0; sub < nsub; ++sub) merge_ml(m, l, s_fold[sub * R + threadIdx.x][0], s_fold[sub * R + threadIdx.x][1]);
+    s_m[threadIdx.x] = m;
+    s_iz[threadIdx.x] = 1.f / l;
+  }
+  __syncthreads();
+  float best[2] = {-INFINITY, -INFINITY};
+  for (int g = 0; g < G; ++g) {
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    auto add4 = [&](int n, const v8 (&x)[4]) {
+      const int r0 = g * W + 16 * n + 4 * wave;
+      float m[4], iz[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        m[j] = s_m[r0 + j];
+        iz[j] = s_iz[r0 + j];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = fin_prob<RM>(base2_logit<RM>((float)x[j][e]), m[j], iz[j]);
+        acc[e] += (p[0] + p[1]) + (p[2] + p[3]);
+      }
+    };
+    for (int n = 0; n < W / 16; n += 2) {
+      if (g > 0 || n > 0) {
+        rows4(g, n, xa);
+        if (n + 1 < W / 16) rows4(g, n + 1, xb);
+      }
+      add4(n, xa);
+      if (n + 1 < W / 16) add4(n + 1, xb);
+    }
+    f32x4* d = reinterpret_cast<f32x4*>(&s_a[wave][8 * lane]);
+    d[0] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    d[1] = f32x4{acc[4], acc[5], acc[6], acc[7]};
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = (int)threadIdx.x + 256 * q, ti = o0 - 8 + i;
+      s_sum[i] = ti >= 0 && ti < span ? round_fixed<RM>((s_a[0][i] + s_a[1][i]) + (s_a[2][i] + s_a[3][i])) : pad;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = (int)threadIdx.x + 256 * q;
+      if (i >= kFcOut) continue;
+      float v = fc_pool<POOL, P>(s_sum, 8 + i);
+      if constexpr (POOL == 0) v = v / (float)(2 * P + 1);
+      best[q] = fmaxf(best[q], round_fixed<RM>(v));
+    }
+  }
+  float* o = S + (int64_t)job * span;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = (int)threadIdx.x + 256 * q;
+    if (i < kFcOut && o0 + i < span) o[o0 + i] = accumulate ? o[o0 + i] + best[q] : best[q];
   }
 }
 
@@ -1630,12 +1943,22 @@ static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 // Query sets below this many rows take the logit-store path.
 constexpr int kLogitRows = 32;
 
+// Summed windows of whole 16-row tiles under the cast chain take it up to
+// kCastLogitRows rows, with 16-bit logits.
+bool cast_window_logits(int G, int W, int flags) {
+  const int R = G * W;
+  return (flags & (HC_SCORE_ROUND_BF16 | HC_SCORE_ROUND_F16)) && (flags & HC_SCORE_SUM_WINDOW) && W % 16 == 0 &&
+         R >= kLogitRows && R <= kCastLogitRows;
+}
+
 size_t score_workspace_bytes(int njobs, int L, int G, int W, int flags) {
   const int R = G * W;
   const int nchunks = (L + kScoreChunk - 1) / kScoreChunk;
   const int wout = (flags & HC_SCORE_SUM_WINDOW) ? 1 : W;
-  const size_t tail = R < kLogitRows ? (size_t)njobs * R * L * sizeof(float)          // logits
-                                     : (size_t)njobs * wout * G * L * sizeof(float);  // probabilities
+  size_t tail = R < kLogitRows ? (size_t)njobs * R * L * sizeof(float)          // logits
+                               : (size_t)njobs * wout * G * L * sizeof(float);  // probabilities
+  if (R < kLogitRows || cast_window_logits(G, W, flags))
+    tail = std::max(tail, (size_t)njobs * R * (size_t)cast_logit_pitch(L) * 2);
   return align256((size_t)njobs * nchunks * R * 2 * sizeof(float)) +
          align256((size_t)njobs * R * 2 * sizeof(float)) + align256(tail);
 }
@@ -1772,7 +2095,11 @@ static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* 
   float* A = reinterpret_cast<float*>(reinterpret_cast<char*>(stats) + align256((size_t)njobs * a.R * 2 * sizeof(float)));
   const size_t qbytes = (size_t)a.NT * 16 * kQPitch * sizeof(T);
   const size_t lds1 = qbytes + (size_t)kScoreWaves * a.NT * 16 * 2 * sizeof(float);
-  const bool via_logits = a.R < kLogitRows;
+  const bool pool57 = kernel == 5 || kernel == 7;
+  // (Whole windows of keys in the store are not summed by any caller.)
+  const bool cast_window = !STORE && pool57 && cast_window_logits(a.G, a.W, a.flags) &&
+                           (a.R <= kLogitRows || (int64_t)njobs * a.R * cast_logit_pitch(a.span) * 2 <= kCastLogitBytes);
+  const bool via_logits = a.R < kLogitRows || cast_window;
   const int rm = (a.flags & HC_SCORE_ROUND_BF16) ? 1 : (a.flags & HC_SCORE_ROUND_F16) ? 2 : 0;
   int nparts = 0;  // statistics partials per job: the stats grid's x extent
   if (!STORE && via_logits && a.R <= 16) {
@@ -1806,33 +2133,66 @@ static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* 
   int rc = check_launch("hc_score(stats)");
   if (rc) return rc;
   // The logit path's finish folds the partials itself, unless the merge
-  // launch also has the histograms to clear.
-  const bool fold_in_finish = via_logits && !hist;
+  // launch also has the histograms to clear, or every tile of a window would
+  // read more partials than logits.
+  const bool fold_in_finish = via_logits && !hist && !(cast_window && nparts > 2 * kFcLoad / 16);
   if (!fold_in_finish) {
     hipLaunchKernelGGL(score_stats_merge_kernel, dim3((njobs * a.R + 3) / 4), dim3(256), 0, s, part, nparts, a.R,
                        njobs, stats, hist, hist ? (int64_t)njobs * wout * kKeyDigitBins : (int64_t)0);
     if ((rc = check_launch("hc_score(merge)"))) return rc;
   }
   const float* fpart = fold_in_finish ? part : nullptr;
+  const int acc_out = (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, sum_out = (a.flags & HC_SCORE_SUM_WINDOW) ? 1 : 0;
+  if (via_logits && rm != 0 && pool57 && !hist) {
+    if (a.span > 0) {
+      const int ntiles = (a.span + kFcOut - 1) / kFcOut;
+      // Several tiles a workgroup where there are more than kFcGrid of them:
+      // each folds the row statistics once.
+      const int64_t per = cast_window ? 1 : ((int64_t)ntiles * njobs * wout + kFcGrid - 1) / kFcGrid;
+      const dim3 cgrid((unsigned)((ntiles + per - 1) / per), njobs * wout);
+#define HC_FCAST(RM, PL, P)                                                                                        \
+  do {                                                                                                            \
+    if (cast_window)                                                                                              \
+      hipLaunchKernelGGL((score_finish_window_kernel<RM, PL, P>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts, \
+                         a.R, a.G, a.W, a.span, acc_out, scores);                                                 \
+    else                                                                                                          \
+      hipLaunchKernelGGL((score_finish_cast_kernel<RM, PL, P>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts,   \
+                         a.R, a.G, a.W, a.span, sum_out, acc_out, scores);                                        \
+  } while (0)
+#define HC_FCAST_P(RM, PL)       \
+  do {                           \
+    if (kernel == 5)             \
+      HC_FCAST(RM, PL, 2);       \
+    else                         \
+      HC_FCAST(RM, PL, 3);       \
+  } while (0)
+      if (rm == 1) { if (pooling == 0) HC_FCAST_P(1, 0); else HC_FCAST_P(1, 1); }
+      else { if (pooling == 0) HC_FCAST_P(2, 0); else HC_FCAST_P(2, 1); }
+#undef HC_FCAST_P
+#undef HC_FCAST
+      if ((rc = check_launch("hc_score(finish)"))) return rc;
+    }
+    return HC_OK;
+  }
   if (via_logits) {
     if (a.span > 0) {
-      const bool reg_pool = kernel == 5 || kernel == 7;
+      const bool reg_pool = pool57;
       const int ntiles = (a.span + (reg_pool ? kFinRegTile : kFinTile) - 1) / (reg_pool ? kFinRegTile : kFinTile);
       const int rows = njobs * wout;
       const int ht = reg_pool ? kFinRegHistTiles : kFinHistTiles;
       const int per_row = hist ? (ntiles + ht - 1) / ht : ntiles;
       const dim3 fgrid(per_row, rows);
-      const int sum_w = (a.flags & HC_SCORE_SUM_WINDOW) ? 1 : 0;
+      const int sum_w = sum_out;
       const int rmode = rm;
 #define HC_FINISH2(RM, PL, HI)                                                                              \
   do {                                                                                                      \
-    if (kernel == 5)                                                                                        \
-      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, HI, 2>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
+    if (kernel == 5 && (RM == 0 || HI))                                                                     \
+      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, (RM != 0 || HI), 2>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
                          nparts, a.R,                                                                 \
                          a.G, a.W, a.span, sum_w, kernel, (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, scores,    \
                          hist);                                                                             \
-    else if (kernel == 7)                                                                                   \
-      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, HI, 3>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
+    else if (kernel == 7 && (RM == 0 || HI))                                                                \
+      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, (RM != 0 || HI), 3>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
                          nparts, a.R,                                                                 \
                          a.G, a.W, a.span, sum_w, kernel, (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, scores,    \
                          hist);                                                                             \

@@ -88,6 +88,37 @@ def test_bf16_cast_chain(dev):
     assert (s == ref).mean() >= 0.97
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("G,W,L,keep", [
+    (1, 32, 33, True),     # one scored position
+    (1, 32, 528, True),    # exactly one tile of 496 outputs, two chunks and a bit of keys
+    (1, 32, 529, False), (1, 64, 1559, True), (2, 16, 1025, False), (1, 48, 997, True), (2, 32, 260, True),
+    (4, 16, 2500, True),
+    (1, 32, 17000, True),  # more partials than a tile's logits: the merge launch
+    # fewer than 32 rows: one wave per query head, four heads at a time
+    (1, 1, 1, False), (4, 1, 496, False), (5, 1, 497, False), (7, 1, 1489, False), (9, 1, 505, False),
+    (3, 4, 1000, False), (2, 8, 991, True), (1, 16, 513, True)])
+@pytest.mark.parametrize("pooling,kernel", [("avgpool", 5), ("maxpool", 7)])
+def test_cast_chain_16bit_logits(dev, dt, G, W, L, keep, pooling, kernel):
+    """Scores under the cast chain, whose logits are stored in 16 bits, over
+    tile edges, window sizes and group sizes.  A 32-bit sum on the other side
+    of a rounding edge moves a score by one unit of the type at each of the
+    chain's last two roundings: 2 * 2^-7 relative in bfloat16, 2 * 2^-10 in
+    float16, whose subnormal unit is 2^-24."""
+    Hkv, dtype = 3, TORCH_DT[dt]
+    q, k = qk(dev, 1, Hkv * G, Hkv, W + 3, max(L, W), dtype, 11 + L + W)
+    L = k.shape[2]
+    s = as_np(compress.window_scores(q, k, range(Hkv), G, W, pooling, kernel, window_keep=keep, round_dtype=dtype))
+    qn, kn = as_np(q), as_np(k)
+    qw = np.stack([qn[0, h * G:(h + 1) * G, -W:] for h in range(Hkv)])
+    ref = O.window_scores(qw, kn[0], pooling, kernel, window_keep=keep,
+                          io_dtype="bfloat16" if dt == "bf16" else "float16")
+    assert s.shape == ref.shape
+    unit, floor = (2.0 ** -7, 0.0) if dt == "bf16" else (2.0 ** -10, 2.0 ** -24)
+    assert (np.abs(s - ref) <= 2 * (unit * np.abs(ref) + floor)).all()
+    assert (s == ref).mean() >= 0.9
+
+
 def test_pivot_step_scores_read_store_in_place(dev):
     B, Hq, Hkv, L, S, G = 1, 32, 8, 2500, 5, 4
     q, k = qk(dev, B, Hq, Hkv, 1, L, torch.bfloat16, 5, strided=False)
