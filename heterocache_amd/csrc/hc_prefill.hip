@@ -442,15 +442,16 @@ __global__ __launch_bounds__(kPfThreads, sizeof(T) == 4 ? 1 : 3) void prefill_at
 // ---------------------------------------------------------------------------
 constexpr int kDvPitch = HC_TILE + 8;            // fp32: transposed V row, 32 k-slots + skew
 constexpr int kDvNPitch = HC_HEAD_DIM + 16;      // 16-bit: natural V row, 128 channels + skew
+constexpr int kDvKPitch = HC_HEAD_DIM + 8;       // 16-bit: natural K row; 16 rows' equal chunks fall on distinct banks
 constexpr int kDvWaves = 4;
 constexpr float kDvLazy = 8.f;                   // lazy-rescale threshold, log2 units
 
-// Per-wave V buffer (elements): fp32 keeps the tile transposed ([channel][k-slot]);
-// 16-bit types keep it in natural layout ([token][channel]) and read the A
-// operand with the LDS transpose read.
+// Per-wave buffer (elements): fp32 keeps the V tile transposed
+// ([channel][k-slot]); 16-bit types keep V and K tiles in natural layout
+// ([token][channel]) and read V's A operand with the LDS transpose read.
 template <typename T>
 constexpr int dv_wave_elems() {
-  return sizeof(T) == 4 ? HC_HEAD_DIM * kDvPitch : HC_TILE * kDvNPitch;
+  return sizeof(T) == 4 ? HC_HEAD_DIM * kDvPitch : HC_TILE * (kDvNPitch + kDvKPitch);
 }
 template <typename T>
 constexpr size_t dv_lds_bytes() {
@@ -503,18 +504,30 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
   const T* vb = reinterpret_cast<const T*>(a.v) + b * a.v_sb + kvh * a.v_sh;
   const int tile0 = split * d.tps + wave, tile_end = min(split * d.tps + d.tps, d.ntiles);
 
-  // K: A operand rows = tokens t0 + 16h + n16, k-slots = channels 32s + 8*g4 + [0, 8).
-  // V: chunk c = lane + 64i of the tile = token c / 16, channels 8*(c % 16) + [0, 8).
-  auto load_tile = [&](int tile, vec8 (&kr)[2][4], vec8 (&vr)[8]) {
+  // K and V: chunk c = lane + 64i of the tile = token c / 16, channels
+  // 8*(c % 16) + [0, 8), so a load reads four whole 256-byte rows.  fp32 K is
+  // read as the A operand: rows = tokens t0 + 16h + n16, k-slots = channels
+  // 32s + 8*g4 + [0, 8).  (16-bit K read so, 16 rows of 64 bytes a load:
+  // 48.1 us for one query over 65541 keys, 8 KV heads, against 45.6 now.)
+  constexpr bool kKInLds = sizeof(T) == 2;
+  T* const skv = sv + HC_TILE * kDvNPitch;
+  // Keys past Lk are read from the last one (clamped, branch-free loads);
+  // their logits are masked.
+  auto load_tile = [&](int tile, vec8 (&kr)[8], vec8 (&vr)[8]) {
     const int t0 = tile * HC_TILE;
+    if constexpr (kKInLds) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int t = t0 + 16 * h + n16;
-      // Keys past Lk are read from the last one (clamped, branch-free
-      // loads); their logits are masked.
-      const T* p = kb + (int64_t)min(t, a.Lk - 1) * a.k_st + 8 * g4;
+      for (int i = 0; i < 8; ++i) {
+        const int c = lane + 64 * i, t = t0 + (c >> 4);
+        kr[i] = load8_stream<T>(kb + (int64_t)min(t, a.Lk - 1) * a.k_st + 8 * (c & 15));
+      }
+    } else {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kr[h][s] = load8_stream<T>(p + 32 * s);
+      for (int h = 0; h < 2; ++h) {
+        const T* p = kb + (int64_t)min(t0 + 16 * h + n16, a.Lk - 1) * a.k_st + 8 * g4;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) kr[4 * h + s] = load8_stream<T>(p + 32 * s);
+      }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -529,7 +542,7 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
   for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
-  auto step = [&](int tile, const vec8 (&kr)[2][4], const vec8 (&vr)[8]) {
+  auto step = [&](int tile, const vec8 (&kr)[8], const vec8 (&vr)[8]) {
     const int t0 = tile * HC_TILE;
     if constexpr (sizeof(T) == 4) {
       // V tile -> transposed LDS rows: channel 8*(c%16) + e, k-slot of token c/16.
@@ -549,12 +562,26 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
         *reinterpret_cast<vec8*>(sv + (c >> 4) * kDvNPitch + 8 * (c & 15)) = vr[i];
       }
     }
+    if constexpr (kKInLds) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int c = lane + 64 * i;
+        *reinterpret_cast<vec8*>(skv + (c >> 4) * kDvKPitch + 8 * (c & 15)) = kr[i];
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      __builtin_amdgcn_wave_barrier();
+    }
     // S^T = K Q^T: rows = tokens t0 + 16h + 4*g4 + j, column n16.
     f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) sacc[h] = mma_16x16x32(kr[h][s], qop[s], sacc[h]);
+      for (int s = 0; s < 4; ++s) {
+        if constexpr (kKInLds)
+          sacc[h] = mma_16x16x32(load8(skv + (16 * h + n16) * kDvKPitch + 32 * s + 8 * g4), qop[s], sacc[h]);
+        else
+          sacc[h] = mma_16x16x32(kr[4 * h + s], qop[s], sacc[h]);
+      }
     if (t0 + HC_TILE - 1 > shift) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -614,7 +641,7 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
     __builtin_amdgcn_wave_barrier();
   };
 
-  vec8 ka[2][4], va_[8], kb2[2][4], vb2[8];
+  vec8 ka[8], va_[8], kb2[8], vb2[8];
   int tile = tile0;
   if (tile < tile_end) load_tile(tile, ka, va_);
   while (tile < tile_end) {
@@ -672,65 +699,78 @@ __global__ __launch_bounds__(kDvWaves * 64, sizeof(T) == 4 ? 1 : 2) void prefill
 }
 
 // Split partials of one query -> its output row (and, for the last st_rows
-// queries, its statistics): one workgroup per (batch, query head, query) of
-// kMergeGroups x 128 threads, thread (group, d) summing channel d over the
-// splits s = group (mod kMergeGroups).  The splits' maximum and weights
-// 2^(m_s - M) are formed once, cooperatively, into LDS, so each thread's sum
-// is a run of independent loads; the groups' sums are added in LDS.  Splits
-// with no visible key (m = -inf) add nothing.
+// queries, its statistics): one workgroup per (batch, query head, query) and
+// kMergeSlice channels, thread (group, d) taking channel d of the splits
+// s = group (mod kMergeGroups).  The merge is bound by latency: the loads of
+// kBatch splits are issued unconditionally (addresses clamped into the row,
+// values masked after), fold in registers, and the groups are combined once
+// through LDS.  Splits with no visible key (m = -inf) add nothing.  (One
+// workgroup per query that first folded the splits' maximum, then their
+// weights, then the channels took a round of loads for each: 7.2 us for 32 queries of 64 splits, 4.0
+// now.)
 constexpr int kPfMaxSplits = 1024;
-constexpr int kMergeGroups = 4;
-constexpr int kMergeThreads = kMergeGroups * HC_HEAD_DIM;
-template <typename T>
+constexpr int kMergeThreads = 256;
+template <typename T, int kMergeSlice>
 __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(const PfArgs a) {
-  __shared__ float s_w[kPfMaxSplits];
-  __shared__ float s_red[kMergeThreads / 64];
-  __shared__ float s_acc[kMergeGroups][HC_HEAD_DIM];
+  constexpr int kMergeGroups = kMergeThreads / kMergeSlice;
+  constexpr int kBatch = 8;
+  __shared__ float s_m[kMergeGroups], s_l[kMergeGroups];
+  __shared__ float s_o[kMergeGroups][kMergeSlice];
   const int64_t qx = blockIdx.x;  // (b * Hq + hq) * Lq + qi
+  const int dl = threadIdx.x % kMergeSlice, grp = threadIdx.x / kMergeSlice;
+  const int d = blockIdx.y * kMergeSlice + dl;
+  const float* pp = a.part + qx * a.nsplit * kPfPartStride;
+  float m = -INFINITY, l = 0.f, acc = 0.f;
+  for (int s0 = grp; s0 < a.nsplit; s0 += kBatch * kMergeGroups) {
+    float x[kBatch], ms[kBatch], ls[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const float* p = pp + (int64_t)min(s0 + k * kMergeGroups, a.nsplit - 1) * kPfPartStride;
+      x[k] = p[d];
+      ms[k] = p[HC_HEAD_DIM];
+      ls[k] = p[HC_HEAD_DIM + 1];
+    }
+    float mn = m;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      if (s0 + k * kMergeGroups >= a.nsplit) ms[k] = -INFINITY;
+      mn = fmaxf(mn, ms[k]);
+    }
+    if (mn == -INFINITY) continue;
+    const float f = fast_exp2(m - mn);
+    l *= f;
+    acc *= f;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const float e = fast_exp2(ms[k] - mn);
+      if (e > 0.f) {
+        l = fmaf(ls[k], e, l);
+        acc = fmaf(x[k], e, acc);
+      }
+    }
+    m = mn;
+  }
+  if (dl == 0) {
+    s_m[grp] = m;
+    s_l[grp] = l;
+  }
+  s_o[grp][dl] = acc;
+  __syncthreads();
+  if (grp != 0) return;
+  float M = -INFINITY, L = 0.f, sum = 0.f;
+#pragma unroll
+  for (int g = 0; g < kMergeGroups; ++g) M = fmaxf(M, s_m[g]);
+#pragma unroll
+  for (int g = 0; g < kMergeGroups; ++g) {
+    const float e = s_m[g] == -INFINITY ? 0.f : fast_exp2(s_m[g] - M);
+    if (e > 0.f) {
+      L = fmaf(s_l[g], e, L);
+      sum = fmaf(s_o[g][dl], e, sum);
+    }
+  }
   const int qi = (int)(qx % a.Lq);
   const int bh = (int)(qx / a.Lq);
   const int hq = bh % a.Hq, b = bh / a.Hq;
-  const float* pp = a.part + qx * a.nsplit * kPfPartStride;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int d = tid % HC_HEAD_DIM, grp = tid / HC_HEAD_DIM;
-  constexpr int nw = kMergeThreads / 64;
-  float mloc = -INFINITY;
-  for (int s = tid; s < a.nsplit; s += kMergeThreads) mloc = fmaxf(mloc, pp[s * kPfPartStride + HC_HEAD_DIM]);
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) mloc = fmaxf(mloc, __shfl_xor(mloc, off, 64));
-  if (lane == 0) s_red[wv] = mloc;
-  __syncthreads();
-  float M = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < nw; ++w) M = fmaxf(M, s_red[w]);
-  __syncthreads();  // s_red is reused below
-  float lloc = 0.f;
-  for (int s = tid; s < a.nsplit; s += kMergeThreads) {
-    const float ms = pp[s * kPfPartStride + HC_HEAD_DIM];
-    const float e = ms == -INFINITY ? 0.f : fast_exp2(ms - M);
-    s_w[s] = e;
-    if (e > 0.f) lloc = fmaf(pp[s * kPfPartStride + HC_HEAD_DIM + 1], e, lloc);
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) lloc += __shfl_xor(lloc, off, 64);
-  if (lane == 0) s_red[wv] = lloc;
-  __syncthreads();
-  float L = 0.f;
-#pragma unroll
-  for (int w = 0; w < nw; ++w) L += s_red[w];
-  float acc = 0.f;
-#pragma unroll 8
-  for (int s = grp; s < a.nsplit; s += kMergeGroups) {
-    const float e = s_w[s];
-    const float x = pp[s * kPfPartStride + d];
-    acc = e > 0.f ? fmaf(x, e, acc) : acc;
-  }
-  s_acc[grp][d] = acc;
-  __syncthreads();
-  if (grp != 0) return;
-  float sum = 0.f;
-#pragma unroll
-  for (int g = 0; g < kMergeGroups; ++g) sum += s_acc[g][d];
   T* o = reinterpret_cast<T*>(a.out) + b * a.o_sb + hq * a.o_sh + (int64_t)qi * a.o_st;
   o[d] = Elem<T>::from_f32(sum / L);
   const int w = qi - (a.Lq - a.st_rows);
@@ -739,6 +779,21 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(const PfAr
     so[0] = M;
     so[1] = L;
   }
+}
+
+// Slices of 16 channels while their workgroups are all resident at once;
+// with more queries (short chunks) the device is full anyway, and one
+// workgroup per query reads each (m, l) once.
+constexpr int64_t kMergeSlicedGrid = 2048;
+template <typename T>
+int launch_merge(const PfArgs& a, hipStream_t stream) {
+  const int64_t nq = (int64_t)(a.rows / a.Hkv) * a.Hq * a.Lq;
+  if (nq * (HC_HEAD_DIM / 16) <= kMergeSlicedGrid)
+    hipLaunchKernelGGL((prefill_merge_kernel<T, 16>), dim3((unsigned)nq, HC_HEAD_DIM / 16), dim3(kMergeThreads), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((prefill_merge_kernel<T, HC_HEAD_DIM>), dim3((unsigned)nq), dim3(kMergeThreads), 0, stream, a);
+  return check_launch("hc_prefill_attn(merge)");
 }
 
 template <typename T>
@@ -764,11 +819,7 @@ int launch_prefill(const PfArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((prefill_attn_kernel<T, false>), dim3((unsigned)grid), dim3(kPfThreads), pf_lds_bytes<T>(),
                        stream, a);
   if ((rc = check_launch("hc_prefill_attn"))) return rc;
-  if (a.nsplit > 1) {
-    const int64_t nq = (int64_t)(a.rows / a.Hkv) * a.Hq * a.Lq;
-    hipLaunchKernelGGL((prefill_merge_kernel<T>), dim3((unsigned)nq), dim3(kMergeThreads), 0, stream, a);
-    rc = check_launch("hc_prefill_attn(merge)");
-  }
+  if (a.nsplit > 1) rc = launch_merge<T>(a, stream);
   return rc;
 }
 
@@ -786,9 +837,7 @@ int launch_decode_shaped(const DvArgs& d, hipStream_t stream) {
                      d);
   int rc = check_launch("hc_prefill_attn(decode-shaped)");
   if (rc) return rc;
-  const int64_t nq = (int64_t)(d.a.rows / d.a.Hkv) * d.a.Hq * d.a.Lq;
-  hipLaunchKernelGGL((prefill_merge_kernel<T>), dim3((unsigned)nq), dim3(kMergeThreads), 0, stream, d.a);
-  return check_launch("hc_prefill_attn(merge)");
+  return launch_merge<T>(d.a, stream);
 }
 
 // Resident workgroups of the decode-shaped kernel on the current device.

@@ -270,6 +270,8 @@ DECODE_SHAPED_CASES = [
     (2, 28, 4, 2, 5000),      # GQA 7, two queries: 14 columns, batch 2
     (1, 8, 8, 16, 3001),      # no GQA, 16 queries, a ragged last tile
     (3, 4, 2, 8, 1100),       # GQA 2 x 8 queries, batch 3
+    (4, 32, 32, 16, 1030),    # more queries than the sliced merge takes
+    (1, 4, 1, 1, 4129),       # one KV row, a tile of one key
 ]
 
 
