@@ -12,20 +12,27 @@
 // rule: equal scores keep the lower position first.
 //
 // Multi-workgroup radix select: every job is cut into 4096-position chunks,
-// one 256-thread workgroup per (chunk, job), six launches per call:
-//  1-4. select_hist_kernel(pass p): histogram of the 8-bit digit p (MSB
+// one 256-thread workgroup per (chunk, job), one launch per 8-bit digit and
+// one for the output:
+//  1..n. select_hist_kernel(pass p): histogram of the 8-bit digit p (MSB
 //       first) of the order-preserving uint32 keys that match the digits
-//       already fixed, per wave in LDS, summed into a global per-job
-//       histogram.  Each workgroup recovers the fixed digits by replaying
-//       the picks on the earlier global histograms (one wave-wide scan each).
-//  5.   select_count_kernel: replays all four picks -> the exact key tau of
-//       the last kept element and how many elements equal to tau are kept;
-//       counts per chunk the keys above tau and equal to tau.
-//  6.   select_write_kernel: chunk bases from the per-chunk counts, then an
-//       ordered compaction (ballot ranks inside each 64-position row, LDS
-//       scan across rows), so the output is ascending by construction.  It
-//       also clears the global histograms for the next call and writes the
-//       force-kept window tail.
+//       already fixed, per wave in LDS.  All passes but the last sum it into
+//       a global per-job histogram, from which the next pass's workgroups
+//       recover the fixed digits by replaying the picks (one wave-wide scan
+//       each).  The last pass leaves each chunk's histogram in the scratch
+//       buffer instead, with the count of the chunk's keys above the fixed
+//       digits: the chunks' sum gives the exact key tau of the last kept
+//       element, the sum over the chunks before one its output base.
+//  n+1. select_write_kernel: sums those, then an ordered compaction (ballot
+//       ranks inside each 64-position row, a wave scan across rows), so the
+//       output is ascending by construction.  It also clears the global
+//       histograms for the next call and writes the force-kept window tail.
+// Each launch costs about 5 us however little it does, so a launch less is
+// what counts: 8 rows of 128K, 16 key bits, 24.1 us in four launches (hist 2 x
+// 4.8, count 5.9, write 8.5) -> 18.5 in three (2 x 4.8, write 9.0).  A workgroup
+// sums 1 KB per chunk: for rows of more than kSelFoldChunks chunks, where that
+// grows beyond what a launch costs, select_count_kernel counts each chunk's
+// keys above and equal to tau instead.
 #include <algorithm>
 
 #include "hc_common.h"
@@ -39,6 +46,7 @@ constexpr int kSelChunk = 4096;                      // positions per workgroup
 constexpr int kSelRows = kSelChunk / kSelThreads;    // 16 rows of 256 positions
 constexpr int kSelBins = 256;
 constexpr int kSelMaxChunks = 4096;
+constexpr int kSelFoldChunks = 64;  // longest row whose output pass sums its chunks' histograms
 constexpr int kSelSub = 1;    // LDS sub-histograms per wave (power of two)
 
 struct SelJob {
@@ -55,6 +63,23 @@ __device__ __forceinline__ SelJob sel_job(const int32_t* caps, int job, int span
   const int body = min(window > 0 ? max(cap - window, 0) : cap, span);
   j.body = min(body, (int)max((int64_t)0, idx_stride - window));
   return j;
+}
+
+// Inclusive prefix sum of one value per thread across a workgroup of NT.
+template <int NT>
+__device__ __forceinline__ int block_inclusive_scan(int v, int* s_tmp) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  if (lane == 63) s_tmp[wave] = v;
+  __syncthreads();
+  int add = 0;
+  for (int w = 0; w < wave; ++w) add += s_tmp[w];
+  __syncthreads();
+  return v + add;
 }
 
 struct SelState {
@@ -109,12 +134,26 @@ __device__ __forceinline__ SelState sel_replay(const unsigned* __restrict__ ghis
   return st;
 }
 
+// FOLD: the last pass; state[job] = {fixed digits, elements still to keep},
+// chist[job][chunk] = {the digit's kSelBins counts, keys above the fixed digits}.
+constexpr int kSelChunkWords = kSelBins + 1;
+template <bool FOLD>
 __global__ __launch_bounds__(kSelThreads) void select_hist_kernel(const float* __restrict__ scores,
                                                                   int64_t score_stride, int span,
                                                                   const int32_t* __restrict__ caps, int window,
                                                                   int64_t idx_stride, unsigned* __restrict__ ghist,
-                                                                  int pass) {
+                                                                  int pass, int* __restrict__ state,
+                                                                  int* __restrict__ chist) {
   const int job = blockIdx.y, chunk = blockIdx.x;
+  // The scores first: in flight over the budget's and the histograms' reads.
+  const float* s = scores + (int64_t)job * score_stride;
+  const int t0 = chunk * kSelChunk;
+  float v[kSelRows];
+#pragma unroll
+  for (int r = 0; r < kSelRows; ++r) {
+    const int t = t0 + r * kSelThreads + threadIdx.x;
+    v[r] = t < span ? s[t] : 0.f;
+  }
   const SelJob jb = sel_job(caps, job, span, window, idx_stride);
   if (jb.body <= 0 || jb.body >= span) return;
   // kSelSub histograms per wave (lane % kSelSub) spread same-bin atomics.
@@ -124,16 +163,9 @@ __global__ __launch_bounds__(kSelThreads) void select_hist_kernel(const float* _
   const SelState st = sel_replay(gh, jb.body, pass, s_pick);
   for (int i = threadIdx.x; i < kSelWaves * kSelSub * kSelBins; i += kSelThreads) (&s_hist[0][0])[i] = 0;
   __syncthreads();
-  const float* s = scores + (int64_t)job * score_stride;
-  const int t0 = chunk * kSelChunk;
   const int shift = 24 - 8 * pass;
   unsigned* wh = s_hist[(threadIdx.x >> 6) * kSelSub + (threadIdx.x & (kSelSub - 1))];
-  float v[kSelRows];
-#pragma unroll
-  for (int r = 0; r < kSelRows; ++r) {
-    const int t = t0 + r * kSelThreads + threadIdx.x;
-    v[r] = t < span ? s[t] : 0.f;
-  }
+  int above = 0;
 #pragma unroll
   for (int r = 0; r < kSelRows; ++r) {
     const int t = t0 + r * kSelThreads + threadIdx.x;
@@ -145,6 +177,28 @@ __global__ __launch_bounds__(kSelThreads) void select_hist_kernel(const float* _
     // readlane / ballot rounds, was slower on clustered pooled scores:
     // 0.067 against 0.050 ms for 8 rows of 128K, top 49629.)
     if (valid) atomicAdd(&wh[d], 1u);
+    if constexpr (FOLD) above += t < span && (u & st.mask) > st.prefix;
+  }
+  if constexpr (FOLD) {
+    __shared__ int s_above[kSelWaves];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) above += __shfl_xor(above, off, 64);
+    if ((threadIdx.x & 63) == 0) s_above[threadIdx.x >> 6] = above;
+    __syncthreads();
+    int* ch = chist + ((int64_t)job * gridDim.x + chunk) * kSelChunkWords;
+    static_assert(kSelThreads == kSelBins, "one bin a thread");
+    unsigned c = 0;
+#pragma unroll
+    for (int w = 0; w < kSelWaves * kSelSub; ++w) c += s_hist[w][threadIdx.x];
+    ch[threadIdx.x] = (int)c;
+    if (threadIdx.x == 0) {
+      ch[kSelBins] = (s_above[0] + s_above[1]) + (s_above[2] + s_above[3]);
+      if (chunk == 0) {
+        state[job * 4] = (int)st.prefix;
+        state[job * 4 + 1] = st.k_rem;
+      }
+    }
+    return;
   }
   __syncthreads();
   for (int b = threadIdx.x; b < kSelBins; b += kSelThreads) {
@@ -163,11 +217,10 @@ __global__ __launch_bounds__(kSelThreads) void select_count_kernel(const float* 
                                                                    const unsigned* __restrict__ ghist,
                                                                    int* __restrict__ state, int* __restrict__ cnt,
                                                                    int32_t* __restrict__ counts, int nchunks,
-                                                                   int32_t* __restrict__ zero_out, int npass) {
+                                                                   int npass) {
   const int job = blockIdx.y, chunk = blockIdx.x;
   const SelJob jb = sel_job(caps, job, span, window, idx_stride);
   if (chunk == 0 && threadIdx.x == 0 && counts) counts[job] = jb.body + jb.tail;
-  if (chunk == 0 && threadIdx.x == 0 && zero_out) zero_out[job] = 0;
   if (jb.body <= 0 || jb.body >= span) return;
   __shared__ int s_pick[3];
   __shared__ int s_red[2][kSelWaves];
@@ -214,21 +267,56 @@ __global__ __launch_bounds__(kSelThreads) void select_count_kernel(const float* 
   }
 }
 
+// FOLD: after select_hist_kernel<true> (pass npass - 1); otherwise state and
+// cnt are select_count_kernel's.
+template <bool FOLD>
 __global__ __launch_bounds__(kSelThreads) void select_write_kernel(const float* __restrict__ scores,
                                                                    int64_t score_stride, int span,
                                                                    const int32_t* __restrict__ caps, int window,
                                                                    int32_t* __restrict__ idx, int64_t idx_stride,
                                                                    unsigned* __restrict__ ghist,
                                                                    const int* __restrict__ state,
-                                                                   const int* __restrict__ cnt, int nchunks) {
+                                                                   const int* __restrict__ cnt, int nchunks,
+                                                                   int32_t* __restrict__ counts, int npass) {
   const int job = blockIdx.y, chunk = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t0 = chunk * kSelChunk;
+  // Every read first, so that they are in flight together (a row whose budget
+  // is none or all of it uses none of them; an unwritten scratch is then read).
+  const float* s = scores + (int64_t)job * score_stride;
+  float v[kSelRows];
+#pragma unroll
+  for (int r = 0; r < kSelRows; ++r) {
+    const int t = t0 + r * kSelThreads + tid;
+    v[r] = t < span ? s[t] : 0.f;
+  }
+  // FOLD: this thread's digit, in descending order: its count in all chunks
+  // and in the chunks before this one.
+  const int d = kSelBins - 1 - tid;
+  int tot = 0, before = 0, g = 0;
+  if constexpr (FOLD) {
+    constexpr int kBatch = 32;
+    const int* ch = cnt + (int64_t)job * nchunks * kSelChunkWords;
+    if (tid < chunk) g = ch[tid * kSelChunkWords + kSelBins];
+    static_assert(kSelFoldChunks <= kSelThreads, "one chunk's count a thread");
+    for (int c0 = 0; c0 < nchunks; c0 += kBatch) {
+      int x[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) x[i] = ch[min(c0 + i, nchunks - 1) * kSelChunkWords + d];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        tot += c0 + i < nchunks ? x[i] : 0;
+        before += c0 + i < chunk ? x[i] : 0;
+      }
+    }
+  }
+  const int st0 = state[job * 4], k_rem = state[job * 4 + 1], st2 = state[job * 4 + 2];
   const SelJob jb = sel_job(caps, job, span, window, idx_stride);
   int32_t* out = idx + (int64_t)job * idx_stride;
-  const int t0 = chunk * kSelChunk;
   if (chunk == 0) {
     for (int i = tid; i < jb.tail; i += kSelThreads) out[jb.body + i] = span + i;
     for (int i = tid; i < 4 * kSelBins; i += kSelThreads) ghist[(int64_t)job * 4 * kSelBins + i] = 0u;
+    if (FOLD && tid == 0 && counts) counts[job] = jb.body + jb.tail;
   }
   if (jb.body <= 0) return;
   if (jb.body >= span) {
@@ -237,84 +325,103 @@ __global__ __launch_bounds__(kSelThreads) void select_write_kernel(const float* 
     return;
   }
   __shared__ int s_base[2];
-  __shared__ int s_cnt[2][kSelRows][kSelWaves];
-  __shared__ int s_off[2][kSelRows][kSelWaves];
-  const uint32_t tau = (uint32_t)state[job * 4];
-  const int need_eq = state[job * 4 + 1];
-  const bool all_ties = state[job * 4 + 2] != 0;
-  if (wave == 0) {
-    // Kept elements and ties in the chunks before this one: G keys above tau
-    // and EQ ties in all, of which the ties taken in position order number
-    // min(max(need_eq, 0), EQ) (the chunk-by-chunk sum of
-    // max(0, min(e_c, need_eq - ties before c)) telescopes to it).  Summed
-    // by the 64 lanes: one thread walking the chunks took a round trip per
-    // few chunks, ~8 us for the last chunk of a 128K row.
-    int g = 0, e = 0;
-    for (int c = lane; c < chunk; c += 64) {
-      g += cnt[((int64_t)job * nchunks + c) * 2];
-      e += cnt[((int64_t)job * nchunks + c) * 2 + 1];
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      g += __shfl_xor(g, off, 64);
-      e += __shfl_xor(e, off, 64);
-    }
-    if (lane == 0) {
-      s_base[0] = g + (all_ties ? e : min(max(need_eq, 0), e));
-      s_base[1] = e;
-    }
-  }
-  const float* s = scores + (int64_t)job * score_stride;
+  __shared__ int s_cnt[2][kSelRows * kSelWaves];
   uint32_t keys[kSelRows];
 #pragma unroll
-  for (int r = 0; r < kSelRows; ++r) {
-    const int t = t0 + r * kSelThreads + tid;
-    keys[r] = t < span ? order_key(s[t]) : 0u;
+  for (int r = 0; r < kSelRows; ++r) keys[r] = order_key(v[r]);  // used below span only
+  uint32_t tau;
+  int need_eq;
+  bool all_ties;
+  if constexpr (FOLD) {
+    __shared__ int s_tmp[kSelWaves], s_pick[3], s_g[kSelWaves];
+    const int above = block_inclusive_scan<kSelThreads>(tot, s_tmp) - tot;
+    if (above < k_rem && above + tot >= k_rem) {
+      s_pick[0] = d;
+      s_pick[1] = k_rem - above;
+      s_pick[2] = tot;
+      s_base[1] = before;
+    }
+    __syncthreads();
+    tau = (uint32_t)st0 | (uint32_t)s_pick[0] << (32 - 8 * npass);
+    need_eq = s_pick[1];
+    all_ties = s_pick[2] == need_eq;
+    if (d > s_pick[0]) g += before;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) g += __shfl_xor(g, off, 64);
+    if (lane == 0) s_g[wave] = g;
+    __syncthreads();
+    if (tid == 0) {
+      const int e = s_base[1];
+      s_base[0] = (s_g[0] + s_g[1]) + (s_g[2] + s_g[3]) + (all_ties ? e : min(need_eq, e));
+    }
+  } else {
+    tau = (uint32_t)st0;
+    need_eq = k_rem;
+    all_ties = st2 != 0;
+    if (wave == 0) {
+      // Kept elements and ties in the chunks before this one: G keys above tau
+      // and EQ ties in all, of which the ties taken in position order number
+      // min(max(need_eq, 0), EQ) (the chunk-by-chunk sum of
+      // max(0, min(e_c, need_eq - ties before c)) telescopes to it).  Summed
+      // by the 64 lanes: one thread walking the chunks took a round trip per
+      // few chunks, ~8 us for the last chunk of a 128K row.
+      int g = 0, e = 0;
+      for (int c = lane; c < chunk; c += 64) {
+        g += cnt[((int64_t)job * nchunks + c) * 2];
+        e += cnt[((int64_t)job * nchunks + c) * 2 + 1];
+      }
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        g += __shfl_xor(g, off, 64);
+        e += __shfl_xor(e, off, 64);
+      }
+      if (lane == 0) {
+        s_base[0] = g + (all_ties ? e : min(max(need_eq, 0), e));
+        s_base[1] = e;
+      }
+    }
   }
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  // Entries in the chunk's rows before (row r, this wave): every wave scans
+  // the kSelRows x kSelWaves counts, one a lane.  (One thread walking them
+  // took 2 x 64 dependent LDS reads.)
+  static_assert(kSelRows * kSelWaves == 64, "one count a lane");
+  auto row_starts = [&](int which) {
+    const int v = s_cnt[which][lane];
+    int incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int y = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += y;
+    }
+    return incl - v;
+  };
   // Ties: ranks of equal keys in position order (row-major over (row, wave)).
   uint64_t eqm[kSelRows];
 #pragma unroll
   for (int r = 0; r < kSelRows; ++r) {
     const int t = t0 + r * kSelThreads + tid;
     eqm[r] = __ballot(t < span && keys[r] == tau);
-    if (lane == 0) s_cnt[1][r][wave] = __popcll(eqm[r]);
+    if (lane == 0) s_cnt[1][r * kSelWaves + wave] = __popcll(eqm[r]);
   }
   __syncthreads();
-  if (tid == 0) {
-    int e = s_base[1];
-    for (int r = 0; r < kSelRows; ++r)
-      for (int w = 0; w < kSelWaves; ++w) {
-        s_off[1][r][w] = e;
-        e += s_cnt[1][r][w];
-      }
-  }
-  __syncthreads();
+  const int eq_starts = s_base[1] + row_starts(1);
   uint64_t selm[kSelRows];
 #pragma unroll
   for (int r = 0; r < kSelRows; ++r) {
     const int t = t0 + r * kSelThreads + tid;
     bool take = t < span && keys[r] > tau;
-    if (t < span && keys[r] == tau) {
-      const int rank = s_off[1][r][wave] + __popcll(eqm[r] & below);
-      take = all_ties || rank < need_eq;
-    }
+    const int start = __shfl(eq_starts, r * kSelWaves + wave, 64);
+    if (t < span && keys[r] == tau) take = all_ties || start + __popcll(eqm[r] & below) < need_eq;
     selm[r] = __ballot(take);
-    if (lane == 0) s_cnt[0][r][wave] = __popcll(selm[r]);
+    if (lane == 0) s_cnt[0][r * kSelWaves + wave] = __popcll(selm[r]);
   }
   __syncthreads();
-  if (tid == 0) {
-    int p = s_base[0];
-    for (int r = 0; r < kSelRows; ++r)
-      for (int w = 0; w < kSelWaves; ++w) {
-        s_off[0][r][w] = p;
-        p += s_cnt[0][r][w];
-      }
-  }
-  __syncthreads();
+  const int starts = s_base[0] + row_starts(0);
 #pragma unroll
   for (int r = 0; r < kSelRows; ++r) {
-    if ((selm[r] >> lane) & 1ull) out[s_off[0][r][wave] + __popcll(selm[r] & below)] = t0 + r * kSelThreads + tid;
+    const int start = __shfl(starts, r * kSelWaves + wave, 64);
+    if ((selm[r] >> lane) & 1ull) out[start + __popcll(selm[r] & below)] = t0 + r * kSelThreads + tid;
   }
 }
 
@@ -420,23 +527,6 @@ __global__ __launch_bounds__(kDriftHistThreads) void drift_hist_kernel(const flo
   uint32_t* o = hist + (int64_t)blockIdx.y * kKeyDigitBins;
   for (int b = threadIdx.x; b < kKeyDigitBins; b += kDriftHistThreads)
     if (h[b]) atomicAdd(&o[b], h[b]);
-}
-
-// Inclusive prefix sum of one value per thread across a workgroup of NT.
-template <int NT>
-__device__ __forceinline__ int block_inclusive_scan(int v, int* s_tmp) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(v, d, 64);
-    if (lane >= d) v += u;
-  }
-  if (lane == 63) s_tmp[wave] = v;
-  __syncthreads();
-  int add = 0;
-  for (int w = 0; w < wave; ++w) add += s_tmp[w];
-  __syncthreads();
-  return v + add;
 }
 
 // The bin of an NBINS histogram where the count, accumulated in scan order
@@ -772,7 +862,7 @@ size_t select_hist_bytes(int njobs) { return (size_t)njobs * 4 * kSelBins * size
 
 size_t select_scratch_bytes(int njobs, int span) {
   const int nchunks = (span + kSelChunk - 1) / kSelChunk;
-  return (size_t)njobs * (4 * sizeof(int) + (size_t)nchunks * 2 * sizeof(int));
+  return (size_t)njobs * (4 + (size_t)nchunks * (nchunks <= kSelFoldChunks ? kSelChunkWords : 2)) * sizeof(int);
 }
 
 }  // namespace hc
@@ -814,20 +904,25 @@ extern "C" int hc_select_topk(const float* scores, int64_t score_stride, int njo
   int* cnt = state + (size_t)njobs * 4;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(nchunks > 0 ? nchunks : 1, njobs);
-  if (nchunks > 0) {
-    for (int pass = 0; pass < npass; ++pass) {
-      hipLaunchKernelGGL(select_hist_kernel, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps, window,
-                         idx_stride, ghist, pass);
-      int rc = check_launch("hc_select_topk(hist)");
-      if (rc) return rc;
-    }
+  const bool fold = nchunks <= kSelFoldChunks;
+  for (int pass = 0; nchunks > 0 && pass < npass; ++pass) {
+    auto fn = fold && pass == npass - 1 ? select_hist_kernel<true> : select_hist_kernel<false>;
+    hipLaunchKernelGGL(fn, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps, window, idx_stride, ghist,
+                       pass, state, cnt);
+    int rc = check_launch("hc_select_topk(hist)");
+    if (rc) return rc;
+  }
+  if (fold) {
+    hipLaunchKernelGGL(select_write_kernel<true>, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps,
+                       window, idx, idx_stride, ghist, state, cnt, nchunks, counts, npass);
+    return check_launch("hc_select_topk(write)");
   }
   hipLaunchKernelGGL(select_count_kernel, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps, window,
-                     idx_stride, ghist, state, cnt, counts, nchunks, (int32_t*)nullptr, npass);
+                     idx_stride, ghist, state, cnt, counts, nchunks, npass);
   int rc = check_launch("hc_select_topk(count)");
   if (rc) return rc;
-  hipLaunchKernelGGL(select_write_kernel, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps, window,
-                     idx, idx_stride, ghist, state, cnt, nchunks);
+  hipLaunchKernelGGL(select_write_kernel<false>, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps,
+                     window, idx, idx_stride, ghist, state, cnt, nchunks, counts, npass);
   return check_launch("hc_select_topk(write)");
 }
 

@@ -271,6 +271,23 @@ def test_select_window_mode(dev):
     check_select(s, caps, W, as_np(idx).astype(np.int64), as_np(counts).astype(np.int64))
 
 
+@pytest.mark.parametrize("span", [1, 63, 4096, 4097, 131072, 64 * 4096, 64 * 4096 + 1])
+@pytest.mark.parametrize("rounded", [None, torch.bfloat16, torch.float16])
+def test_select_chunk_edges(dev, span, rounded):
+    """One chunk, whole chunks, and the longest row whose output pass sums its
+    chunks' histograms and the next one: bit-exact, ties across chunks
+    included, in two calls (the second finds the histograms cleared)."""
+    rng = np.random.default_rng(span)
+    s = torch.tensor(rng.random((4, span)).astype(np.float32) ** 4)
+    if rounded is not None:
+        s = s.to(rounded).float()
+    s[1] = (s[1] * 8).round() / 8
+    caps = [max(1, span // 3), max(1, span // 2), span - 1, 1]
+    for _ in range(2):
+        idx, counts = compress.select_kept(s.to(dev), caps, round_dtype=rounded)
+        check_select(s.numpy(), caps, 0, as_np(idx).astype(np.int64), as_np(counts).astype(np.int64))
+
+
 def test_select_all_equal_scores(dev):
     s = np.full((2, 3000), 0.125, np.float32)
     idx, counts = compress.select_kept(torch.tensor(s).to(dev), [1500, 7])
