@@ -48,6 +48,7 @@ SIGNATURES = {
     "hc_decode_num_parts": (c_int64, [c_void_p, c_int, c_int]),
     "hc_decode_chunk_tiles": (c_int, [c_int, c_void_p, c_int, c_int]),
     "hc_decode_workspace_size": (c_size_t, [c_int, c_int, c_int64]),
+    "hc_decode_plan": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
     "hc_gather_store": (c_int, [c_int, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int,
                                 c_void_p, c_void_p]),

@@ -114,6 +114,16 @@ def decode_chunk_tiles(host_row_len, group, dtype):
     return n
 
 
+def decode_plan(host_row_len, group, dtype, added):
+    """(chunk_tiles, parts, workspace bytes) of a decode launch over rows of
+    host_row_len[r] + added tokens (added: 0 or 1)."""
+    lens = _lens_i32(host_row_len)
+    plan = (_lib.c_int64 * 3)()
+    _lib.check(_lib.load().hc_decode_plan(dtype_code(dtype), lens.ctypes.data, len(lens), int(group), added,
+                                          ctypes.addressof(plan)))
+    return plan[0], plan[1], plan[2]
+
+
 def decode_attn(q, kstore, vstore, row_tile_off, row_len, host_row_len, scale, out=None, row_order=None,
                 k_new=None, v_new=None, chunk_tiles=None, stream=None, workspace=None, num_parts=None,
                 row_cap=None, status=None, stat_len=0, stat_out=None, stat_flags=0):
@@ -161,7 +171,6 @@ def decode_attn(q, kstore, vstore, row_tile_off, row_len, host_row_len, scale, o
             raise TypeError("k_new/v_new must share q's dtype")
         k_new = k_new.contiguous()
         v_new = v_new.contiguous()
-        host_row_len = _lens_i32(host_row_len) + np.int32(1)
     if row_order is not None and (row_order.dtype != torch.int32 or row_order.numel() != rows):
         raise ValueError("row_order must be an int32 permutation of the rows")
     q = q.contiguous()
@@ -169,14 +178,19 @@ def decode_attn(q, kstore, vstore, row_tile_off, row_len, host_row_len, scale, o
         out = torch.empty_like(q)
     elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous() or out.device != q.device:
         raise ValueError("out must be a contiguous tensor of q's shape, dtype and device")
+    added = 0 if k_new is None else 1
+    nbytes = None
     if chunk_tiles is None:
-        chunk_tiles = decode_chunk_tiles(host_row_len, G, q.dtype)
-    nparts = decode_num_parts(host_row_len, chunk_tiles)
+        chunk_tiles, nparts, nbytes = decode_plan(host_row_len, G, q.dtype, added)
+    else:
+        nparts = decode_num_parts(_lens_i32(host_row_len) + np.int32(added), chunk_tiles)
     if num_parts is not None:
         if int(num_parts) < nparts:
             raise ValueError(f"num_parts {num_parts} is below the {nparts} parts these lengths need")
         nparts = int(num_parts)
-    nbytes = lib.hc_decode_workspace_size(rows, G, nparts)
+        nbytes = None
+    if nbytes is None:
+        nbytes = lib.hc_decode_workspace_size(rows, G, nparts)
     ws = workspace if workspace is not None else WORKSPACE.get(q.device, nbytes)
     st_ptr = _ptr(status) if k_new is not None else None
     if stat_len:

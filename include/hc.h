@@ -159,6 +159,10 @@ int64_t hc_decode_num_parts(const int32_t* host_row_len, int rows, int chunk_til
  * its split internally). */
 int hc_decode_chunk_tiles(int dtype, const int32_t* host_row_len, int rows, int group);
 size_t hc_decode_workspace_size(int rows, int group, int64_t num_parts);
+/* The three above for lengths host_row_len[r] + added (0 or 1, a fused append)
+ * in one call: chunk_parts_bytes[0..2] = chunk size, parts, workspace bytes. */
+int hc_decode_plan(int dtype, const int32_t* host_row_len, int rows, int group, int added,
+                   int64_t* chunk_parts_bytes);
 
 /*
  * Gather natural-layout rows into store slots [0, count[j]) of row dst_row[j]:

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 import torch
 
+from heterocache_amd import _lib, ops
 from heterocache_amd.store import KVStore
 from oracle import hc_oracle as O
 from tests.gpu_util import ATTN_TOL, TORCH_DT, as_np, fill_store
@@ -434,3 +435,17 @@ def test_graph_replay_past_capacity_raises_oom(dev):
     assert torch.equal(snap[0][0], after[0][0]) and torch.equal(snap[0][1], after[0][1])
     with pytest.raises(RuntimeError, match="Layer 3 OOM."):
         gst.check_status()
+
+
+@pytest.mark.parametrize("rows", [1, 8, 128, 129])
+@pytest.mark.parametrize("added", [0, 1])
+def test_decode_plan_equals_its_parts(dev, rows, added):
+    """hc_decode_plan: the chunk size, part count and workspace bytes of the
+    three calls it stands for, on the lengths a fused append leaves."""
+    lens = np.random.default_rng(rows).integers(0, 70000, rows).astype(np.int32)
+    chunk, parts, nbytes = ops.decode_plan(lens, 4, torch.bfloat16, added)
+    assert chunk == ops.decode_chunk_tiles(lens + np.int32(added), 4, torch.bfloat16)
+    assert parts == ops.decode_num_parts(lens + np.int32(added), chunk)
+    assert nbytes == _lib.load().hc_decode_workspace_size(rows, 4, parts)
+    with pytest.raises(_lib.HCError, match="negative length"):
+        ops.decode_plan(np.full(rows, -2, np.int32), 4, torch.bfloat16, added)
