@@ -152,8 +152,10 @@ class H2OKVCluster:
         self.merge = merge
 
     def heavy_hitter_scores(self, key_states, query_states):
-        """[B*H, L] float32: sum over every query position of its softmax row."""
-        return ops.attn_column_sums(query_states, key_states, 1.0 / math.sqrt(query_states.shape[-1]))
+        """[B*H, L] float32: sum over every query position of its softmax row
+        (over the first B batches, H heads and L tokens of the keys)."""
+        B, H = query_states.shape[:2]
+        return ops.attn_column_sums(query_states, key_states[:B, :H], 1.0 / math.sqrt(query_states.shape[-1]))
 
     def update_kv(self, key_states, query_states, value_states, attention_mask, num_key_value_groups):
         assert key_states.shape[-2] == query_states.shape[-2]

@@ -619,12 +619,24 @@ def score_given_stats(q, q_off, q_head_stride, q_row_stride, kstore, row_tile_of
 def attn_column_sums(q, k, scale, out=None, stream=None):
     """[B*H, L] float32: per key, the softmax probability it takes from every
     query position of its head, summed (no mask; hc_attn_column_sums in
-    include/hc.h).  q, k: [B, H, L, 128], the first L keys of k."""
-    lib = _lib.load()
-    _require_cuda(q, k, out)
+    include/hc.h).  q: [B, H, L, 128]; k: [B, H, >= L, 128], of which the
+    first L keys count.  With `stream` the whole call, its copies and
+    allocations included, runs on that stream."""
+    if q.dim() != 4 or k.dim() != 4 or q.shape[3] != HEAD_DIM or k.shape[3] != HEAD_DIM:
+        raise ValueError(f"q {tuple(q.shape)}, k {tuple(k.shape)}: both must be [B, H, L, {HEAD_DIM}]")
+    B, H, L, _ = q.shape
+    if k.shape[:2] != q.shape[:2] or k.shape[2] < L:
+        raise ValueError(f"q {tuple(q.shape)}, k {tuple(k.shape)}: k must hold the batches and heads of q "
+                         "(GQA keys repeated per query head) and at least its tokens")
     if q.dtype != k.dtype:
         raise TypeError("q and k must share a dtype")
-    B, H, L, _ = q.shape
+    _require_cuda(q, k, out)
+    if k.device != q.device or (out is not None and out.device != q.device):
+        raise ValueError("q, k and out must be on one device")
+    if stream is not None:
+        with torch.cuda.stream(stream):
+            return attn_column_sums(q, k, scale, out=out)
+    lib = _lib.load()
     if out is None:
         out = torch.empty((B * H, L), dtype=torch.float32, device=q.device)
     elif out.dtype != torch.float32 or out.numel() < B * H * L or not out.is_contiguous():
@@ -633,16 +645,19 @@ def attn_column_sums(q, k, scale, out=None, stream=None):
         return out
     if k.stride(2) < HEAD_DIM or k.stride(2) % 8:
         raise ValueError(f"key token stride {k.stride(2)}")
-    # The kernels read rows in 16-byte units: other layouts are copied first.
-    per16 = 16 // q.element_size()
-    q, k = (t if t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(
+    # The kernels read rows in 16-byte units, 64 of them from one 32-bit
+    # offset: other layouts are copied first.
+    esz = q.element_size()
+    per16, max_tok = 16 // esz, (1 << 31) // (64 * esz)
+    k = k[:, :, :L]
+    q, k = (t if t.stride(3) == 1 and t.data_ptr() % 16 == 0 and (L == 1 or t.stride(2) < max_tok) and all(
         n == 1 or st % per16 == 0 for n, st in zip(t.shape[:3], t.stride())) else
         t.clone(memory_format=torch.contiguous_format) for t in (q, k))
     strides = np.array([[st if n > 1 else 0 for n, st in zip(t.shape[:3], t.stride())] for t in (q, k)], dtype=np.int64)
     code = dtype_code(q.dtype)
     ws = torch.empty(lib.hc_attn_column_sums_workspace(code, B, H, L), dtype=torch.uint8, device=q.device)
     _lib.check(lib.hc_attn_column_sums(code, _ptr(q), strides.ctypes.data, _ptr(k), strides.ctypes.data + 24, B, H, L,
-                                       float(scale), _ptr(out), _ptr(ws), ws.numel(), _stream(stream, q)))
+                                       float(scale), _ptr(out), _ptr(ws), ws.numel(), _stream(None, q)))
     return out
 
 

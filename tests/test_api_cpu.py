@@ -1,13 +1,13 @@
 """Reference-API surface that needs no kernel: the baseline caches' legacy
-converters, HeteroCache.clear_temp_kv_cache, and the prefill attention's
-refusal of inputs hc_prefill_attn does not take (CPU only)."""
+converters, HeteroCache.clear_temp_kv_cache, and the refusals of
+inputs that the prefill attention and the column sums do not take (CPU only)."""
 import json
 import os
 
 import pytest
 import torch
 
-from heterocache_amd import llama_model, utils
+from heterocache_amd import kv_cluster, llama_model, ops, utils
 from heterocache_amd.cache_utils import (BaseKVCache, CompressionCacheConfig, HeteroCache, HeteroCacheConfig,
                                          SnapKVCache)
 
@@ -77,3 +77,22 @@ def test_prefill_attention_refuses_padding_and_host_tensors():
         llama_model.prefill_attention(q, q, q, causal.expand(B, 1, L, L), 1.0)
     with pytest.raises(NotImplementedError, match="ROCm device"):
         llama_model.prefill_attention(q, q, q, None, 1.0)
+
+
+@pytest.mark.parametrize("q,k", [
+    ((1, 8, 40, 128), (1, 2, 40, 128)),    # GQA keys, not repeated per query head
+    ((2, 4, 40, 128), (1, 4, 40, 128)),    # a batch too few
+    ((1, 4, 40, 128), (1, 4, 39, 128)),    # a token too few
+    ((1, 4, 40, 128), (1, 5, 40, 128)),
+    ((1, 4, 40, 64), (1, 4, 40, 64)),      # head_dim
+    ((1, 4, 40, 128), (1, 4, 40, 64)),
+    ((4, 40, 128), (4, 40, 128))])
+def test_column_sums_refuse_shapes_they_would_read_past(q, k):
+    """Keys that do not cover the queries' batches, heads and tokens, or rows
+    of another head_dim, are refused before any device work."""
+    q, k = torch.zeros(q), torch.zeros(k)
+    with pytest.raises(ValueError, match=r"must be \[B, H, L, 128\]|must hold the batches and heads"):
+        ops.attn_column_sums(q, k, 0.1)
+    if q.dim() == 4 and k.shape[1] <= q.shape[1]:
+        with pytest.raises(ValueError, match=r"must be \[B, H, L, 128\]|must hold the batches and heads"):
+            kv_cluster.H2OKVCluster().heavy_hitter_scores(k, q)

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from heterocache_amd import ops
+from heterocache_amd import kv_cluster, ops
 from oracle import hc_oracle as O
 from tests.gpu_util import as_np
 
@@ -62,6 +62,50 @@ def test_layouts_that_are_copied(dev):
     _check(q, k)
     with pytest.raises(ValueError):
         ops.attn_column_sums(q, q, SCALE)  # keys: token stride not a multiple of 8
+
+
+def test_longer_and_wider_keys(dev):
+    """Keys of more tokens than the queries count up to the queries' length;
+    the cluster takes the first heads of keys that have more of them."""
+    L = 100
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(2, 3, L, 128, generator=g).half().to(dev)
+    k = torch.randn(3, 5, L + 30, 128, generator=g).half().to(dev)
+    want = ops.attn_column_sums(q, k[:2, :3, :L].contiguous(), SCALE)
+    assert torch.equal(ops.attn_column_sums(q, k[:2, :3], SCALE), want)
+    assert torch.equal(kv_cluster.H2OKVCluster().heavy_hitter_scores(k, q), want)
+
+
+def test_token_stride_past_32_bit_offsets(dev):
+    """64 token strides of 2^31 bytes or more: copied first."""
+    g = torch.Generator().manual_seed(8)
+    flat = torch.zeros(2 * (1 << 24) + 128, dtype=torch.float16, device=dev)
+    k = flat.as_strided((1, 1, 3, 128), (0, 0, 1 << 24, 1))
+    k.copy_(torch.randn(1, 1, 3, 128, generator=g))
+    q = torch.randn(1, 1, 3, 128, generator=g).half().to(dev)
+    _check(q, k)
+    assert torch.equal(ops.attn_column_sums(k, q, SCALE), ops.attn_column_sums(k.contiguous(), q, SCALE))
+
+
+def test_copies_run_on_the_given_stream(dev):
+    """Keys off 16 bytes, written on the call's stream behind a queue of other
+    work: the copy that aligns them waits for them."""
+    L = 200
+    g = torch.Generator().manual_seed(9)
+    flat = torch.zeros(1 + 2 * L * 128, dtype=torch.float16, device=dev)
+    k = flat[1:].view(1, 2, L, 128)
+    src = torch.randn(1, 2, L, 128, generator=g).half().to(dev)
+    q = torch.randn(1, 2, L, 128, generator=g).half().to(dev)
+    big = torch.randn(4096, 4096, device=dev)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        for _ in range(20):
+            big = big @ big * 1e-4
+        k.copy_(src)
+    got = ops.attn_column_sums(q, k, SCALE, stream=s)
+    s.synchronize()
+    assert torch.equal(got, ops.attn_column_sums(q, src, SCALE))
 
 
 def test_infinite_and_nan_rows(dev):
