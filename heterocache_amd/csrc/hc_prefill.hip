@@ -942,9 +942,10 @@ extern "C" size_t hc_prefill_workspace_size(int dtype, int batch, int kv_heads, 
 
 static size_t pf_align256(size_t x) { return (x + 255) / 256 * 256; }
 
-// Split partials after the V tiles: [batch * q_heads * q_len][nsplit][kPfPartStride] floats.
+// Split partials after the V tiles: [batch * q_heads * q_len][nsplit][kPfPartStride]
+// floats.  The decode-shaped kernel writes them for one split as well.
 static size_t pf_part_bytes(int batch, int q_heads, int q_len, int nsplit) {
-  return nsplit > 1 ? (size_t)batch * q_heads * q_len * nsplit * kPfPartStride * sizeof(float) : 0;
+  return (size_t)batch * q_heads * q_len * nsplit * kPfPartStride * sizeof(float);
 }
 
 extern "C" size_t hc_prefill_workspace_bytes(int dtype, int batch, int q_heads, int kv_heads, int q_len,

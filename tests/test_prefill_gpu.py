@@ -297,6 +297,25 @@ def test_prefill_decode_shaped_matches_oracle(dev, dt, case):
     assert np.abs(got - ref).max() <= ATTN_TOL[dt]
 
 
+@pytest.mark.parametrize("dt,case", [("bf16", (33, 16, 8, 1, 1030)), ("f16", (300, 2, 1, 3, 1025)),
+                                     ("f32", (130, 1, 1, 16, 1030)), ("bf16", (1, 300, 300, 1, 3000))])
+def test_prefill_decode_shaped_one_split(dev, dt, case):
+    """More KV rows than half the resident workgroups (256 rows in 16-bit
+    types, 128 in float32) leave one split a row, which still goes through a
+    partial and the merge: the workspace holds those partials, 132 floats per
+    query, behind the V tiles."""
+    B, Hq, Hkv, Lq, Lk = case
+    print(f"prefill_attn decode-shaped one split dt={dt} {case}", flush=True)
+    vt, full = _nbytes(dt, B, Hq, Hkv, Lq, Lk)
+    assert full >= (vt + 255) // 256 * 256 + B * Hq * Lq * 132 * 4
+    q, k, v = _inputs(dev, dt, B, Hq, Hkv, Lq, Lk, 91)
+    scale = 1.0 / math.sqrt(128)
+    got = as_np(ops.prefill_attn(q, k, v, scale))
+    ref = O.prefill_attention(as_np(q), as_np(k), as_np(v), scale)
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() <= ATTN_TOL[dt]
+
+
 def test_prefill_decode_shaped_statistics(dev):
     """Statistics of a decode-shaped call: the oracle's log-normaliser within
     1e-3 (log2 units), the bound within 8 of the row maximum."""
