@@ -1553,14 +1553,17 @@ __global__ __launch_bounds__(256) void score_finish_cast_kernel(const void* __re
 // and job) and their products are replaced by the logits' write and read
 // (2R bytes each).
 // Measured, per call, against two passes over the keys (us): 32 rows, 32 jobs
-// x 8192 keys 39.7 -> 26.6, x 700 18.0 -> 16.6, x 32768 99 -> 86, x 65536 206
-// -> 161; 64 rows, 32 jobs x 8192 50 -> 39, x 16384 (64 MiB of logits) 70 ->
-// 66, 28 jobs x 32768 104 -> 111, 8 jobs x 131072 111 -> 125: the keys still
-// come from the Infinity Cache the second time, and 64 rows of logits are
-// written and read at half their bytes each, so above 32 rows the line lies at
-// kCastLogitBytes.
+// x 700 keys 18.0 -> 16.6, x 8192 39.7 -> 26.6, x 65536 206 -> 162, x 131072
+// (256 MiB of logits) 391 -> 310, 64 jobs x 65536 391 -> 304; 64 rows, 32 jobs
+// x 8192 50 -> 39, x 16384 (64 MiB) 69 -> 65, 28 jobs x 20000 (68 MiB) 72 ->
+// 65, x 32768 (112 MiB) 104 -> 111, 32 jobs x 32768 110 -> 126, 8 jobs x
+// 131072 111 -> 129: the keys still come from the Infinity Cache the second
+// time, and 64 rows of logits are written and read at half their bytes each,
+// so above 32 rows the line lies at kCastLogitBytes.  At 32 rows no loss was
+// found; kCastLogitBytes32, the largest size measured, bounds the workspace.
 constexpr int kCastLogitRows = 64;
 constexpr int64_t kCastLogitBytes = (int64_t)64 << 20;
+constexpr int64_t kCastLogitBytes32 = (int64_t)256 << 20;
 template <int RM, int POOL, int P>
 __global__ __launch_bounds__(256) void score_finish_window_kernel(const void* __restrict__ logits,
                                                                   const float* __restrict__ stats,
@@ -1944,21 +1947,25 @@ static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 constexpr int kLogitRows = 32;
 
 // Summed windows of whole 16-row tiles under the cast chain take it up to
-// kCastLogitRows rows, with 16-bit logits.
-bool cast_window_logits(int G, int W, int flags) {
+// kCastLogitRows rows, with 16-bit logits, while those stay below the limits
+// beside score_finish_window_kernel.  (R below kLogitRows: no such windows.)
+bool cast_window_logits(int njobs, int L, int G, int W, int flags) {
   const int R = G * W;
   return (flags & (HC_SCORE_ROUND_BF16 | HC_SCORE_ROUND_F16)) && (flags & HC_SCORE_SUM_WINDOW) && W % 16 == 0 &&
-         R >= kLogitRows && R <= kCastLogitRows;
+         R >= kLogitRows && R <= kCastLogitRows &&
+         (int64_t)njobs * R * cast_logit_pitch(L) * 2 <= (R == kLogitRows ? kCastLogitBytes32 : kCastLogitBytes);
 }
 
-size_t score_workspace_bytes(int njobs, int L, int G, int W, int flags) {
+// Workspace of a call; window_logits: with the stored logits of
+// cast_window_logits, which a caller's workspace need not hold (the call then
+// reads the keys twice instead).
+size_t score_workspace_bytes(int njobs, int L, int G, int W, int flags, bool window_logits) {
   const int R = G * W;
   const int nchunks = (L + kScoreChunk - 1) / kScoreChunk;
   const int wout = (flags & HC_SCORE_SUM_WINDOW) ? 1 : W;
   size_t tail = R < kLogitRows ? (size_t)njobs * R * L * sizeof(float)          // logits
                                : (size_t)njobs * wout * G * L * sizeof(float);  // probabilities
-  if (R < kLogitRows || cast_window_logits(G, W, flags))
-    tail = std::max(tail, (size_t)njobs * R * (size_t)cast_logit_pitch(L) * 2);
+  if (R < kLogitRows || window_logits) tail = std::max(tail, (size_t)njobs * R * (size_t)cast_logit_pitch(L) * 2);
   return align256((size_t)njobs * nchunks * R * 2 * sizeof(float)) +
          align256((size_t)njobs * R * 2 * sizeof(float)) + align256(tail);
 }
@@ -2085,8 +2092,8 @@ static int launch_probs_pool(ScoreArgs a, int njobs, int pooling, int kernel, St
 }
 
 template <typename T, bool STORE>
-static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* scores, void* ws, uint32_t* hist,
-                        hipStream_t s) {
+static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* scores, void* ws, size_t ws_bytes,
+                        uint32_t* hist, hipStream_t s) {
   const int nchunks = (a.L + kScoreChunk - 1) / kScoreChunk;
   const int wout = (a.flags & HC_SCORE_SUM_WINDOW) ? 1 : a.W;
   float* part = reinterpret_cast<float*>(ws);
@@ -2097,8 +2104,8 @@ static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* 
   const size_t lds1 = qbytes + (size_t)kScoreWaves * a.NT * 16 * 2 * sizeof(float);
   const bool pool57 = kernel == 5 || kernel == 7;
   // (Whole windows of keys in the store are not summed by any caller.)
-  const bool cast_window = !STORE && pool57 && cast_window_logits(a.G, a.W, a.flags) &&
-                           (a.R <= kLogitRows || (int64_t)njobs * a.R * cast_logit_pitch(a.span) * 2 <= kCastLogitBytes);
+  const bool cast_window = !STORE && pool57 && cast_window_logits(njobs, a.L, a.G, a.W, a.flags) &&
+                           ws_bytes >= score_workspace_bytes(njobs, a.L, a.G, a.W, a.flags, true);
   const bool via_logits = a.R < kLogitRows || cast_window;
   const int rm = (a.flags & HC_SCORE_ROUND_BF16) ? 1 : (a.flags & HC_SCORE_ROUND_F16) ? 2 : 0;
   int nparts = 0;  // statistics partials per job: the stats grid's x extent
@@ -2387,7 +2394,8 @@ using namespace hc;
 
 extern "C" size_t hc_score_workspace_size(int njobs, int seq_len, int group, int window, int flags) {
   if (njobs <= 0 || seq_len <= 0 || group <= 0 || window <= 0) return 0;
-  return score_workspace_bytes(njobs, seq_len, group, window, flags);
+  return score_workspace_bytes(njobs, seq_len, group, window, flags,
+                               cast_window_logits(njobs, seq_len, group, window, flags));
 }
 
 extern "C" int hc_score(int dtype, const void* q, const int64_t* q_off, int64_t q_head_stride, int64_t q_row_stride,
@@ -2422,7 +2430,7 @@ extern "C" int hc_score(int dtype, const void* q, const int64_t* q_off, int64_t 
   if (store ? !k_row : !k_off) return set_error(HC_ERR_INVALID, "hc_score: missing key addressing");
   if (!store && (k_tok_stride < HC_HEAD_DIM || (k_tok_stride % 8) != 0))
     return set_error(HC_ERR_INVALID, "hc_score: key token stride %lld", (long long)k_tok_stride);
-  if (workspace_bytes < score_workspace_bytes(njobs, seq_len, group, window, flags))
+  if (workspace_bytes < score_workspace_bytes(njobs, seq_len, group, window, flags, false))
     return set_error(HC_ERR_INVALID, "hc_score: workspace too small");
   if (hist && (R >= kLogitRows || (flags & HC_SCORE_ACCUMULATE)))
     return set_error(HC_ERR_INVALID, "hc_score: a score histogram needs fewer than %d query rows and no accumulation",
@@ -2449,8 +2457,8 @@ extern "C" int hc_score(int dtype, const void* q, const int64_t* q_off, int64_t 
   a.cpw = 1;
   hipStream_t s = (hipStream_t)stream;
 #define HC_SCORE_DISPATCH(T)                                                                          \
-  return store ? launch_score<T, true>(a, njobs, pooling, kernel, scores, workspace, hist, s)         \
-               : launch_score<T, false>(a, njobs, pooling, kernel, scores, workspace, hist, s);
+  return store ? launch_score<T, true>(a, njobs, pooling, kernel, scores, workspace, workspace_bytes, hist, s)  \
+               : launch_score<T, false>(a, njobs, pooling, kernel, scores, workspace, workspace_bytes, hist, s);
   switch (dtype) {
     case HC_DTYPE_BF16: { HC_SCORE_DISPATCH(__bf16) }
     case HC_DTYPE_F16: { HC_SCORE_DISPATCH(_Float16) }

@@ -86,6 +86,7 @@ SELECT_HIST = Workspace()
 # and the query rows below which it can (the logit-store path).
 HIST_BINS = 4096
 HIST_MAX_ROWS = 31
+_ROUND_FLAGS = _lib.HC_SCORE_ROUND_BF16 | _lib.HC_SCORE_ROUND_F16
 
 
 def _lens_i32(host_row_len):
@@ -543,7 +544,10 @@ def score(q, q_off, q_head_stride, q_row_stride, k, k_off, k_tok_stride, seq_len
         _require_cuda(hist)
         if hist.dtype != torch.int32 or not hist.is_contiguous() or hist.numel() < njobs * wout * HIST_BINS:
             raise ValueError(f"hist must be a contiguous int32 tensor of [jobs * W', {HIST_BINS}]")
-    nbytes = lib.hc_score_workspace_size(njobs, seq_len, group, window, flags)
+    # The stored logits of a cast-chain window serve pool kernels 5 and 7 over
+    # natural keys; other calls take the size without a rounding flag.
+    size_flags = flags if kernel in (5, 7) and row_tile_off is None else flags & ~_ROUND_FLAGS
+    nbytes = lib.hc_score_workspace_size(njobs, seq_len, group, window, size_flags)
     ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=q.device)
     pool = {"avgpool": 0, "maxpool": 1}[pooling] if isinstance(pooling, str) else int(pooling)
     _lib.check(lib.hc_score(dtype_code(q.dtype), _ptr(q), _ptr(q_off), int(q_head_stride), int(q_row_stride), _ptr(k),

@@ -381,6 +381,10 @@ int hc_score(int dtype, const void* q, const int64_t* q_off, int64_t q_head_stri
              const int32_t* k_row, int njobs, int seq_len, int group, int window, int flags, int span, int pooling,
              int kernel, float scale, float* scores, void* workspace, size_t workspace_bytes, uint32_t* hist,
              void* stream);
+/* Any call runs in the size without the rounding flags.  With one, summed
+ * windows of 32 to 64 rows get room for 16-bit logits on top while those take
+ * at most 256 MiB (32 rows) or 64 MiB (more): given it, calls over natural
+ * keys with pool kernel 5 or 7 read the keys once instead of twice. */
 size_t hc_score_workspace_size(int njobs, int seq_len, int group, int window, int flags);
 
 /*

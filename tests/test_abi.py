@@ -94,3 +94,23 @@ def test_rounding_flags_are_checked_before_any_launch():
     assert lib.hc_stream_read(fake, 24, fake, 8, None) == _lib.HC_ERR_INVALID
     assert lib.hc_stream_read(fake, 4096, fake, 0, None) == _lib.HC_ERR_INVALID
     assert lib.hc_stream_read(None, 4096, fake, 8, None) == _lib.HC_ERR_INVALID
+
+
+def test_score_workspace_of_cast_windows():
+    """The 16-bit logits of a summed window are asked for while they are at
+    most 64 MiB (256 MiB at 32 rows), and never required; a call of a
+    smaller workspace than the uncast one is refused."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libhc.so not built")
+    lib = _lib.load()
+    fake = 16  # never dereferenced: validation fails first
+    summed, cast = _lib.HC_SCORE_SUM_WINDOW, _lib.HC_SCORE_SUM_WINDOW | _lib.HC_SCORE_ROUND_BF16
+    for jobs, L, W, logits in ((32, 131072, 64, 0), (32, 16384, 64, 64 << 20), (32, 16392, 64, 0),
+                               (32, 131072, 32, 256 << 20), (32, 131080, 32, 0), (64, 131072, 32, 0),
+                               (32, 8192, 48, 24 << 20), (32, 8192, 80, 0)):
+        plain = lib.hc_score_workspace_size(jobs, L, 1, W, summed)
+        size = lib.hc_score_workspace_size(jobs, L, 1, W, cast)
+        assert plain <= size <= plain + logits and (size > plain) == (logits > 0), (jobs, L, W)
+        rc = lib.hc_score(2, fake, fake, 128, 128, fake, fake, 128, None, None, jobs, L, 1, W, cast, L, 0, 5, 0.1, fake,
+                          fake, plain - 1, None, None)
+        assert rc == _lib.HC_ERR_INVALID and b"workspace" in lib.hc_last_error()

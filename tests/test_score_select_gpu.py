@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 import torch
 
-from heterocache_amd import compress, ops
+from heterocache_amd import _lib, compress, ops
 from heterocache_amd.store import KVStore
 from oracle import hc_oracle as O
 from tests.gpu_util import TORCH_DT, as_np
@@ -117,6 +117,38 @@ def test_cast_chain_16bit_logits(dev, dt, G, W, L, keep, pooling, kernel):
     unit, floor = (2.0 ** -7, 0.0) if dt == "bf16" else (2.0 ** -10, 2.0 ** -24)
     assert (np.abs(s - ref) <= 2 * (unit * np.abs(ref) + floor)).all()
     assert (s == ref).mean() >= 0.9
+
+
+@pytest.mark.parametrize("W,L,jobs,stored", [
+    (32, 600, 3, True), (64, 1000, 5, True),
+    (64, 1024, 512, True),    # 64 MiB of logits
+    (64, 1032, 512, False)])  # more: two passes over the keys
+def test_cast_window_workspace(dev, W, L, jobs, stored):
+    """Summed cast windows with the workspace that hc_score_workspace_size
+    asks for and with the one of the uncast call, past whose end nothing is
+    written: both within the chain's tolerance (see
+    test_cast_chain_16bit_logits) of the oracle."""
+    lib, scale = _lib.load(), 1 / math.sqrt(128)
+    q, k = qk(dev, 1, jobs, jobs, W, L, torch.bfloat16, 7 * W + L)
+    flags = _lib.HC_SCORE_SUM_WINDOW | _lib.HC_SCORE_CAUSAL_WINDOW | _lib.HC_SCORE_ROUND_BF16
+    least = lib.hc_score_workspace_size(jobs, L, 1, W, flags & ~_lib.HC_SCORE_ROUND_BF16)
+    full = lib.hc_score_workspace_size(jobs, L, 1, W, flags)
+    assert (full > least) == stored
+    off_q, off_k = (torch.arange(jobs, device=dev) * t.stride(1) for t in (q, k))
+    picks = sorted({0, jobs // 2, jobs - 1})
+    ref = O.window_scores(as_np(q)[0, picks][:, None], as_np(k)[0, picks], "avgpool", 5, window_keep=True,
+                          io_dtype="bfloat16")
+    for size in (least, full):
+        ws = torch.full((full + 4096,), 0x5A, dtype=torch.uint8, device=dev)
+        out = torch.empty((jobs, L - W), dtype=torch.float32, device=dev)
+        _lib.check(lib.hc_score(_lib.HC_DTYPE_BF16, q.data_ptr(), off_q.data_ptr(), q.stride(1), q.stride(2),
+                                k.data_ptr(), off_k.data_ptr(), k.stride(2), None, None, jobs, L, 1, W, flags, L - W, 0,
+                                5, scale, out.data_ptr(), ws.data_ptr(), size, None,
+                                torch.cuda.current_stream().cuda_stream))
+        assert bool((ws[size:] == 0x5A).all())
+        s = as_np(out)[picks]
+        assert (np.abs(s - ref) <= 2 * 2.0 ** -7 * np.abs(ref)).all()
+        assert (s == ref).mean() >= 0.9
 
 
 def test_pivot_step_scores_read_store_in_place(dev):
