@@ -30,10 +30,15 @@
 // Each launch costs about 5 us however little it does, so a launch less is
 // what counts: 8 rows of 128K, 16 key bits, 24.1 us in four launches (hist 2 x
 // 4.8, count 5.9, write 8.5) -> 18.5 in three (2 x 4.8, write 9.0); the whole
-// call 23 -> 18, 350 rows 216 -> 159, 8 rows of 256K 26 -> 22.  A workgroup sums
-// 1 KB per chunk: for rows of more than kSelFoldChunks chunks, where that
-// grows towards the 16 KB of scores it reads, select_count_kernel counts each
-// chunk's keys above and equal to tau instead.
+// call 23 -> 18, 350 rows 216 -> 159, 8 rows of 256K 26 -> 22.  A workgroup
+// reads 1 KB per chunk of its row for that, at 64 chunks four times the 16 KB
+// of scores it reads, where select_count_kernel leaves eight bytes a chunk.
+// Count launch against sums, us a call: 64 chunks, 1 / 8 / 32 / 128 rows 23.5
+// / 24.9 / 45.2 / 144 against 19.2 / 21.7 / 42.2 / 132; 80 and 96 chunks, 8
+// rows 27.1 and 27.8 against 27.0 and 27.4; 98 chunks, 128 rows 218 against
+// 231; 128 chunks, 1 / 8 / 32 rows 25.6 / 30.6 / 84 against 22.2 / 34.0 / 90.
+// So rows of more than kSelFoldChunks chunks keep the count launch (as do
+// calls whose scratch holds no histograms).
 #include <algorithm>
 
 #include "hc_common.h"
@@ -861,9 +866,9 @@ __global__ __launch_bounds__(kSelThreads) void drift_bits_kernel(
 // per-call scratch buffer that needs no initialisation.
 size_t select_hist_bytes(int njobs) { return (size_t)njobs * 4 * kSelBins * sizeof(unsigned); }
 
-size_t select_scratch_bytes(int njobs, int span) {
-  const int nchunks = (span + kSelChunk - 1) / kSelChunk;
-  return (size_t)njobs * (4 + (size_t)nchunks * (nchunks <= kSelFoldChunks ? kSelChunkWords : 2)) * sizeof(int);
+// state and, per chunk, two counts (fold: its histogram and count).
+size_t select_scratch_bytes(int njobs, int nchunks, bool fold) {
+  return (size_t)njobs * (4 + (size_t)nchunks * (fold ? kSelChunkWords : 2)) * sizeof(int);
 }
 
 }  // namespace hc
@@ -877,7 +882,10 @@ extern "C" size_t hc_select_hist_size(int njobs) {
 
 extern "C" size_t hc_select_scratch_size(int njobs, int span) {
   if (njobs <= 0 || span < 0) return 0;
-  return select_scratch_bytes(njobs, span);
+  const int nchunks = (span + kSelChunk - 1) / kSelChunk;
+  // Enough for every shorter span as well, whichever way it is selected.
+  return std::max(select_scratch_bytes(njobs, nchunks, false),
+                  select_scratch_bytes(njobs, std::min(nchunks, kSelFoldChunks), true));
 }
 
 extern "C" int hc_select_topk(const float* scores, int64_t score_stride, int njobs, int span, const int32_t* caps,
@@ -898,14 +906,14 @@ extern "C" int hc_select_topk(const float* scores, int64_t score_stride, int njo
                      (long long)score_stride, (long long)idx_stride);
   const int nchunks = (span + kSelChunk - 1) / kSelChunk;
   if (nchunks > kSelMaxChunks) return set_error(HC_ERR_INVALID, "hc_select_topk: span %d too long", span);
-  if (hist_bytes < select_hist_bytes(njobs) || scratch_bytes < select_scratch_bytes(njobs, span))
+  if (hist_bytes < select_hist_bytes(njobs) || scratch_bytes < select_scratch_bytes(njobs, nchunks, false))
     return set_error(HC_ERR_INVALID, "hc_select_topk: histogram or scratch buffer too small");
   unsigned* ghist = reinterpret_cast<unsigned*>(hist);
   int* state = reinterpret_cast<int*>(scratch);
   int* cnt = state + (size_t)njobs * 4;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(nchunks > 0 ? nchunks : 1, njobs);
-  const bool fold = nchunks <= kSelFoldChunks;
+  const bool fold = nchunks <= kSelFoldChunks && scratch_bytes >= select_scratch_bytes(njobs, nchunks, true);
   for (int pass = 0; nchunks > 0 && pass < npass; ++pass) {
     auto fn = fold && pass == npass - 1 ? select_hist_kernel<true> : select_hist_kernel<false>;
     hipLaunchKernelGGL(fn, grid, dim3(kSelThreads), 0, s, scores, score_stride, span, caps, window, idx_stride, ghist,

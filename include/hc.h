@@ -480,7 +480,10 @@ int hc_select_topk(const float* scores, int64_t score_stride, int njobs, int spa
                    size_t scratch_bytes, int key_bits, void* stream);
 /* hist: hc_select_hist_size(njobs) bytes, zero-filled before its first use;
  * every completed call leaves it zeroed again (calls on one stream may share
- * it).  scratch: hc_select_scratch_size(njobs, span) bytes, no initialisation. */
+ * it).  scratch: hc_select_scratch_size(njobs, span) bytes, no initialisation;
+ * that is enough for any shorter span too.  njobs * (16 + 8 * ceil(span / 4096))
+ * bytes are required: a call of up to 64 such chunks given less than the
+ * asked size takes one launch more. */
 size_t hc_select_hist_size(int njobs);
 size_t hc_select_scratch_size(int njobs, int span);
 

@@ -114,3 +114,23 @@ def test_score_workspace_of_cast_windows():
         rc = lib.hc_score(2, fake, fake, 128, 128, fake, fake, 128, None, None, jobs, L, 1, W, cast, L, 0, 5, 0.1, fake,
                           fake, plain - 1, None, None)
         assert rc == _lib.HC_ERR_INVALID and b"workspace" in lib.hc_last_error()
+
+
+def test_select_scratch_serves_shorter_spans():
+    """hc_select_scratch_size never falls as the span grows (a buffer sized
+    for the longest row serves all), and 16 + 8 bytes a chunk of 4096 per job
+    are all that a call requires."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libhc.so not built")
+    lib = _lib.load()
+    fake = 16  # never dereferenced: validation fails first
+    for jobs in (1, 8):
+        last = 0
+        for span in (0, 1, 4096, 4097, 131072, 64 * 4096, 64 * 4096 + 1, 1 << 20, 4096 * 4096):
+            size = lib.hc_select_scratch_size(jobs, span)
+            least = jobs * (16 + 8 * ((span + 4095) // 4096))
+            assert size >= max(last, least), (jobs, span)
+            last = size
+            rc = lib.hc_select_topk(fake, span, jobs, span, fake, 0, fake, 1, None, fake, 1 << 20, fake, least - 1, 0,
+                                    None)
+            assert rc == _lib.HC_ERR_INVALID and b"scratch" in lib.hc_last_error()

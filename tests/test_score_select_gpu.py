@@ -320,6 +320,29 @@ def test_select_chunk_edges(dev, span, rounded):
         check_select(s.numpy(), caps, 0, as_np(idx).astype(np.int64), as_np(counts).astype(np.int64))
 
 
+@pytest.mark.parametrize("span", [63, 4097, 131072])
+@pytest.mark.parametrize("key_bits", [0, 16])
+def test_select_least_scratch(dev, span, key_bits):
+    """The scratch a call requires, past whose end nothing is written, gives
+    the kept sets of the scratch it asks for."""
+    lib, njobs = _lib.load(), 3
+    rng = np.random.default_rng(span)
+    s = torch.tensor(rng.random((njobs, span)).astype(np.float32) ** 4).bfloat16().float()
+    caps = [max(1, span // 3), span - 1, 1]
+    sd, cd = s.to(dev), torch.tensor(caps, dtype=torch.int32, device=dev)
+    hist = torch.zeros(lib.hc_select_hist_size(njobs), dtype=torch.uint8, device=dev)
+    least = njobs * (16 + 8 * ((span + 4095) // 4096))
+    for size in (least, lib.hc_select_scratch_size(njobs, span)):
+        scratch = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device=dev)
+        idx = torch.empty((njobs, span), dtype=torch.int32, device=dev)
+        counts = torch.empty(njobs, dtype=torch.int32, device=dev)
+        _lib.check(lib.hc_select_topk(sd.data_ptr(), span, njobs, span, cd.data_ptr(), 0, idx.data_ptr(), span,
+                                      counts.data_ptr(), hist.data_ptr(), hist.numel(), scratch.data_ptr(), size,
+                                      key_bits, torch.cuda.current_stream().cuda_stream))
+        assert bool((scratch[size:] == 0x5A).all()) and not hist.any()
+        check_select(s.numpy(), caps, 0, as_np(idx).astype(np.int64), as_np(counts).astype(np.int64))
+
+
 def test_select_all_equal_scores(dev):
     s = np.full((2, 3000), 0.125, np.float32)
     idx, counts = compress.select_kept(torch.tensor(s).to(dev), [1500, 7])
