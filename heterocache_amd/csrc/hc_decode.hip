@@ -24,7 +24,6 @@
 //    tiles) and written into the store by that wave; the merge advances
 //    row_len by one.
 #include <mutex>
-#include <vector>
 
 #include "hc_common.h"
 #include "hc_internal.h"
@@ -690,10 +689,15 @@ constexpr int kDecodeWaves = 4;
 constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
-int64_t decode_num_parts(const int* host_row_len, int rows, int chunk_tiles) {
+// Length of row r with `added` tokens (0 or 1) more, which wraps as int32 does.
+static inline int row_length(const int* host_row_len, int r, int added) {
+  return (int)((uint32_t)host_row_len[r] + (uint32_t)added);
+}
+
+int64_t decode_num_parts(const int* host_row_len, int rows, int chunk_tiles, int added) {
   int64_t total = 0;
   for (int r = 0; r < rows; ++r) {
-    int64_t nt = (host_row_len[r] + HC_TILE - 1) / HC_TILE;
+    int64_t nt = (row_length(host_row_len, r, added) + HC_TILE - 1) / HC_TILE;
     total += nt > 0 ? (nt + chunk_tiles - 1) / chunk_tiles : 1;
   }
   return total;
@@ -801,16 +805,16 @@ static int decode_slots(int dtype, int G) {
 // rounding drops 7-25 % of the workgroups) 22.2 -> 22.8 us, so chunks
 // below kRoundChunk stay as found.
 constexpr int kRoundChunk = 6 * kDecodeWaves;
-static int decode_auto_chunk(const int* host_row_len, int rows, int slots) {
+static int decode_auto_chunk(const int* host_row_len, int rows, int slots, int added) {
   int max_nt = 0;
-  for (int r = 0; r < rows; ++r) max_nt = max(max_nt, (host_row_len[r] + HC_TILE - 1) / HC_TILE);
+  for (int r = 0; r < rows; ++r) max_nt = max(max_nt, (row_length(host_row_len, r, added) + HC_TILE - 1) / HC_TILE);
   if (max_nt <= kDecodeWaves) return kDecodeWaves;
   // One part per row already exceeds the resident slots: one chunk per row.
-  if (decode_num_parts(host_row_len, rows, max_nt) > slots) return max_nt;
+  if (decode_num_parts(host_row_len, rows, max_nt, added) > slots) return max_nt;
   int lo = kDecodeWaves, hi = max_nt;  // parts(chunk) does not increase with chunk
   while (lo < hi) {
     const int mid = lo + (hi - lo) / 2;
-    if (decode_num_parts(host_row_len, rows, mid) <= slots)
+    if (decode_num_parts(host_row_len, rows, mid, added) <= slots)
       hi = mid;
     else
       lo = mid + 1;
@@ -826,17 +830,23 @@ extern "C" size_t hc_decode_workspace_size(int rows, int group, int64_t num_part
   return decode_workspace_bytes_rows(rows, group, num_parts);
 }
 
-extern "C" int hc_decode_chunk_tiles(int dtype, const int32_t* host_row_len, int rows, int group) {
-  clear_error();
+// The chunk size for lengths host_row_len[r] + added, or a negative status.
+static int decode_chunk_tiles(int dtype, const int32_t* host_row_len, int rows, int group, int added) {
   if (dtype != HC_DTYPE_BF16 && dtype != HC_DTYPE_F16 && dtype != HC_DTYPE_F32)
     return set_error(HC_ERR_INVALID, "hc_decode_chunk_tiles: unknown dtype %d", dtype);
   if (rows < 0 || group < 1 || group > 16 || (rows > 0 && !host_row_len))
     return set_error(HC_ERR_INVALID, "hc_decode_chunk_tiles: rows=%d group=%d", rows, group);
   for (int r = 0; r < rows; ++r)
-    if (host_row_len[r] < 0) return set_error(HC_ERR_INVALID, "hc_decode_chunk_tiles: negative length at row %d", r);
+    if (row_length(host_row_len, r, added) < 0)
+      return set_error(HC_ERR_INVALID, "hc_decode_chunk_tiles: negative length at row %d", r);
   const int slots = decode_slots(dtype, group);
   if (slots <= 0) return set_error(HC_ERR_HIP, "hc_decode_chunk_tiles: occupancy query failed");
-  return decode_auto_chunk(host_row_len, rows, slots);
+  return decode_auto_chunk(host_row_len, rows, slots, added);
+}
+
+extern "C" int hc_decode_chunk_tiles(int dtype, const int32_t* host_row_len, int rows, int group) {
+  clear_error();
+  return decode_chunk_tiles(dtype, host_row_len, rows, group, 0);
 }
 
 // One host call for what a launch needs of its lengths: chunk size, part
@@ -848,21 +858,9 @@ extern "C" int hc_decode_plan(int dtype, const int32_t* host_row_len, int rows, 
   clear_error();
   if (rows < 0 || added < 0 || added > 1 || !chunk_parts_bytes || (rows > 0 && !host_row_len))
     return set_error(HC_ERR_INVALID, "hc_decode_plan: rows=%d added=%d", rows, added);
-  int32_t few[128];
-  std::vector<int32_t> many;
-  const int32_t* lens = host_row_len;
-  if (added) {
-    int32_t* sum = few;
-    if (rows > 128) {
-      many.resize(rows);
-      sum = many.data();
-    }
-    for (int r = 0; r < rows; ++r) sum[r] = (int32_t)((uint32_t)host_row_len[r] + 1u);
-    lens = sum;
-  }
-  const int chunk = hc_decode_chunk_tiles(dtype, lens, rows, group);
+  const int chunk = decode_chunk_tiles(dtype, host_row_len, rows, group, added);
   if (chunk <= 0) return chunk;
-  const int64_t parts = decode_num_parts(lens, rows, chunk);
+  const int64_t parts = decode_num_parts(host_row_len, rows, chunk, added);
   chunk_parts_bytes[0] = chunk;
   chunk_parts_bytes[1] = parts;
   chunk_parts_bytes[2] = (int64_t)decode_workspace_bytes_rows(rows, group, parts);

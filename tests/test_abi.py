@@ -5,6 +5,8 @@ CPU only: nothing here launches a kernel.
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -134,3 +136,23 @@ def test_select_scratch_serves_shorter_spans():
             rc = lib.hc_select_topk(fake, span, jobs, span, fake, 0, fake, 1, None, fake, 1 << 20, fake, least - 1, 0,
                                     None)
             assert rc == _lib.HC_ERR_INVALID and b"scratch" in lib.hc_last_error()
+
+
+def test_decode_plan_allocates_nothing():
+    """hc_decode_plan over lengths that one more copy of them would not fit
+    the address space: a status, not an exception out of a C entry."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libhc.so not built")
+    code = """if True:
+        import resource, numpy as np
+        from heterocache_amd import _lib
+        lib, rows = _lib.load(), 1 << 26
+        lens, plan = np.zeros(rows, np.int32), np.zeros(3, np.int64)
+        args = (4, 1, plan.ctypes.data)
+        first = lib.hc_decode_plan(2, lens.ctypes.data, 1, *args)  # the HIP runtime starts outside the limit
+        used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+        resource.setrlimit(resource.RLIMIT_AS, (used + (64 << 20), resource.RLIM_INFINITY))
+        assert lib.hc_decode_plan(2, lens.ctypes.data, rows, *args) == first
+        """
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
