@@ -151,7 +151,10 @@ __global__ __launch_bounds__(kSelThreads) void select_hist_kernel(const float* _
                                                                   int pass, int* __restrict__ state,
                                                                   int* __restrict__ chist) {
   const int job = blockIdx.y, chunk = blockIdx.x;
-  // The scores first: in flight over the budget's and the histograms' reads.
+  const SelJob jb = sel_job(caps, job, span, window, idx_stride);
+  if (jb.body <= 0 || jb.body >= span) return;
+  // The scores first: in flight over the histograms' reads.  (Not over the
+  // budget's, or rows that keep all or none would read them for nothing.)
   const float* s = scores + (int64_t)job * score_stride;
   const int t0 = chunk * kSelChunk;
   float v[kSelRows];
@@ -160,8 +163,6 @@ __global__ __launch_bounds__(kSelThreads) void select_hist_kernel(const float* _
     const int t = t0 + r * kSelThreads + threadIdx.x;
     v[r] = t < span ? s[t] : 0.f;
   }
-  const SelJob jb = sel_job(caps, job, span, window, idx_stride);
-  if (jb.body <= 0 || jb.body >= span) return;
   // kSelSub histograms per wave (lane % kSelSub) spread same-bin atomics.
   __shared__ unsigned s_hist[kSelWaves * kSelSub][kSelBins];
   __shared__ int s_pick[3];
@@ -287,8 +288,20 @@ __global__ __launch_bounds__(kSelThreads) void select_write_kernel(const float* 
   const int job = blockIdx.y, chunk = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int t0 = chunk * kSelChunk;
-  // Every read first, so that they are in flight together (a row whose budget
-  // is none or all of it uses none of them; an unwritten scratch is then read).
+  const SelJob jb = sel_job(caps, job, span, window, idx_stride);
+  int32_t* out = idx + (int64_t)job * idx_stride;
+  if (chunk == 0) {
+    for (int i = tid; i < jb.tail; i += kSelThreads) out[jb.body + i] = span + i;
+    for (int i = tid; i < 4 * kSelBins; i += kSelThreads) ghist[(int64_t)job * 4 * kSelBins + i] = 0u;
+    if (FOLD && tid == 0 && counts) counts[job] = jb.body + jb.tail;
+  }
+  if (jb.body <= 0) return;
+  if (jb.body >= span) {
+    for (int i = tid; i < kSelChunk; i += kSelThreads)
+      if (t0 + i < span) out[t0 + i] = t0 + i;
+    return;
+  }
+  // Every other read now, so that they are in flight together.
   const float* s = scores + (int64_t)job * score_stride;
   float v[kSelRows];
 #pragma unroll
@@ -317,19 +330,6 @@ __global__ __launch_bounds__(kSelThreads) void select_write_kernel(const float* 
     }
   }
   const int st0 = state[job * 4], k_rem = state[job * 4 + 1], st2 = state[job * 4 + 2];
-  const SelJob jb = sel_job(caps, job, span, window, idx_stride);
-  int32_t* out = idx + (int64_t)job * idx_stride;
-  if (chunk == 0) {
-    for (int i = tid; i < jb.tail; i += kSelThreads) out[jb.body + i] = span + i;
-    for (int i = tid; i < 4 * kSelBins; i += kSelThreads) ghist[(int64_t)job * 4 * kSelBins + i] = 0u;
-    if (FOLD && tid == 0 && counts) counts[job] = jb.body + jb.tail;
-  }
-  if (jb.body <= 0) return;
-  if (jb.body >= span) {
-    for (int i = tid; i < kSelChunk; i += kSelThreads)
-      if (t0 + i < span) out[t0 + i] = t0 + i;
-    return;
-  }
   __shared__ int s_base[2];
   __shared__ int s_cnt[2][kSelRows * kSelWaves];
   uint32_t keys[kSelRows];
