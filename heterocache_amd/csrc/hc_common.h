@@ -262,6 +262,26 @@ __device__ __forceinline__ float rows4_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Transpose of four values over the four 16-lane rows of a wave: element j of
+// row i becomes element i of row j (lanes keep their place in the row).
+__device__ __forceinline__ void rows4_transpose(float (&e)[4]) {
+  unsigned u[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) u[j] = __float_as_uint(e[j]);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {  // 2 x 2 blocks: rows 2, 3 of the first with rows 0, 1 of the second
+    const auto s = __builtin_amdgcn_permlane32_swap(u[j], u[j + 2], false, false);
+    u[j] = s[0], u[j + 2] = s[1];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {  // odd rows of the first with even rows of the second
+    const auto s = __builtin_amdgcn_permlane16_swap(u[j], u[j + 1], false, false);
+    u[j] = s[0], u[j + 1] = s[1];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) e[j] = __uint_as_float(u[j]);
+}
+
 // 16 bytes per lane straight from global memory into LDS: lane i's bytes
 // land at lds + 16*i (lds is wave-uniform).
 __device__ __forceinline__ void lds_dma16(const void* src, void* lds) {

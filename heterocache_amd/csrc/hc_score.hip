@@ -371,13 +371,15 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_stats_kernel(ScoreArgs
 // per 256-byte key row, so the pass is bound by streaming the keys -- and
 // the MFMA operand layout of score_stats_kernel makes every wave load touch
 // 16 rows of 64 bytes each.  Here the 16 lanes of group s hold channels
-// 8c..8c+7 (c = lane % 16) of token 8*s + step, so a wave load reads four
-// whole 256-byte token rows, and a lane ends with eight consecutive tokens'
-// logits, stored as whole 16-byte units (eight
-// heads x 128K, four rows: 58.3 -> 53.9 us against scattered float32 stores); the groups' partial dot products of all NR
-// rows are summed by one DPP reduce-scatter (row16_sum_scatter), after which
-// lane c < R of a group holds row c's logit of its token.  Logits are stored as score_stats_kernel stores them (base-2
-// scaled and masked, [job][R][span]) and every workgroup writes one
+// 8c..8c+7 (c = lane % 16) of token 4*step + s, so a wave load reads four
+// whole token rows (1 KB where a head's tokens lie together); the groups'
+// partial dot products of all NR rows are summed by one DPP reduce-scatter
+// (row16_sum_scatter), after which lane c < R of a group holds row c's logit
+// of its token.  A transpose over the groups then gives a lane eight
+// consecutive tokens, so that the logits, in score_stats_kernel's form
+// ([job][R][span], see Logit), leave as 16-byte units (single stores and
+// float32 throughout: 58.3 us for eight heads x 128K, four rows; 53.9 with
+// 16-bit units); every workgroup writes one
 // (max, sum) partial per row, so the merge and finish passes are shared.
 // NR: rows held per lane (R rounded up to 4, 8 or 16).
 constexpr int kRowsSteps = 8;  // 4-token steps per wave and iteration
@@ -461,7 +463,7 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(Score
   auto load_keys = [&](vec8 (&kr)[kRowsSteps], int t0) {
 #pragma unroll
     for (int st = 0; st < kRowsSteps; ++st)
-      kr[st] = load8_stream<T>(kb + (int64_t)min(t0 + kRowsSteps * sub + st, a.L - 1) * a.k_tok_stride);
+      kr[st] = load8_stream<T>(kb + (int64_t)min(t0 + 4 * st + sub, a.L - 1) * a.k_tok_stride);
   };
   auto consume = [&](const vec8 (&kr)[kRowsSteps], int t0) {
     float x[kRowsSteps];
@@ -481,29 +483,39 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_rows_valu_kernel(Score
         acc[r] = d;
       }
       const float mine = row16_sum_scatter<NR>(acc, lane);  // row c % NR
-      const int t = t0 + kRowsSteps * sub + st;
+      const int t = t0 + 4 * st + sub;
       x[st] = t <= limit ? stored_logit<RM>(a, mine) : -INFINITY;
     }
     // The logits are stored after all the iteration's keys are consumed:
     // stores between the key waits count against the same in-order counter,
     // so each wait also waited for the next key (prefill compression 0.192-
     // 0.193 -> 0.191 ms per 128K layer).
-    const int tl = t0 + kRowsSteps * sub;
+    const int tl = t0 + kRowsSteps * sub;  // this lane's first token to store
+    float y[kRowsSteps];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      float e[4] = {x[p], x[2 + p], x[4 + p], x[6 + p]};
+      rows4_transpose(e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[4 * p + i] = e[i];
+    }
     if (owner && tl < a.span) {
-      if (RM != 0 || ((a.span & 3) == 0 && tl + kRowsSteps <= a.span)) {
-        typedef LT __attribute__((ext_vector_type(16 / sizeof(LT)))) lvec;
+      if (RM != 0 || tl + kRowsSteps <= a.span) {
+        // Float32 rows of an odd span start on any word.
         constexpr int kLanes = 16 / sizeof(LT);
+        typedef LT __attribute__((ext_vector_type(kLanes))) lvec;
+        typedef lvec __attribute__((aligned(RM != 0 ? 16 : 4))) lvec_at;
 #pragma unroll
         for (int v = 0; v < kRowsSteps / kLanes; ++v) {
-          lvec y;
+          lvec z;
 #pragma unroll
-          for (int e = 0; e < kLanes; ++e) y[e] = (LT)x[v * kLanes + e];
-          *reinterpret_cast<lvec*>(lrow + tl + v * kLanes) = y;
+          for (int e = 0; e < kLanes; ++e) z[e] = (LT)y[v * kLanes + e];
+          *reinterpret_cast<lvec_at*>(lrow + tl + v * kLanes) = z;
         }
       } else {
 #pragma unroll
-        for (int st = 0; st < kRowsSteps; ++st)
-          if (tl + st < a.span) lrow[tl + st] = (LT)x[st];
+        for (int e = 0; e < kRowsSteps; ++e)
+          if (tl + e < a.span) lrow[tl + e] = (LT)y[e];
       }
     }
 #pragma unroll

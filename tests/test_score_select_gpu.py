@@ -119,6 +119,20 @@ def test_cast_chain_16bit_logits(dev, dt, G, W, L, keep, pooling, kernel):
     assert (s == ref).mean() >= 0.9
 
 
+@pytest.mark.parametrize("G,W,L", [(1, 1, 1), (1, 1, 7), (2, 1, 33), (4, 1, 1001), (1, 8, 1030), (7, 2, 1023), (2, 4, 515)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_few_rows_uncast_odd_spans(dev, G, W, L, dtype):
+    """Float32 logits of a few query rows, whose rows start off 16 bytes where
+    the span is no multiple of four."""
+    Hkv = 3
+    q, k = qk(dev, 1, Hkv * G, Hkv, max(W, 2), max(L, W), dtype, 17 + L + W)
+    s = compress.window_scores(q, k, range(Hkv), G, W, "avgpool", 5)
+    qn, kn = as_np(q), as_np(k)
+    ref = O.window_scores(np.stack([qn[0, h * G:(h + 1) * G, -W:] for h in range(Hkv)]), kn[0], "avgpool", 5,
+                          window_keep=False)
+    assert rel_err(as_np(s), ref) < 2e-4
+
+
 @pytest.mark.parametrize("W,L,jobs,stored", [
     (32, 600, 3, True), (64, 1000, 5, True),
     (64, 1024, 512, True),    # 64 MiB of logits
