@@ -1189,7 +1189,9 @@ __global__ __launch_bounds__(256) void score_finish_kernel(const void* __restric
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int t0 = tile * kFinTile;
     const int tb = t0 + 4 * threadIdx.x;
-    const bool vec_ok = (span & 3) == 0 && tb + 4 <= span;
+    // Rows of 16-bit logits are padded to whole vectors; what is read past
+    // span is not used.
+    const bool vec_in = RMODE != 0 || ((span & 3) == 0 && tb + 4 <= span);
     // Halo: threads [0, p) load t0 - p + x (left), threads [p, 2p) load
     // t0 + kFinTile + (x - p) (right).
     const int th = threadIdx.x < p ? t0 - p + threadIdx.x : t0 + kFinTile + (threadIdx.x - p);
@@ -1212,7 +1214,7 @@ __global__ __launch_bounds__(256) void score_finish_kernel(const void* __restric
             const int r = g * W + w;
             const auto* row = logit_row<RMODE>(logits, (int64_t)job * R + r, span);
             const float m = s_m[r], iz = s_iz[r];
-            if (vec_ok) {
+            if (vec_in) {
               const f32x4 x = read_logits4<RMODE>(row + tb);
 #pragma unroll
               for (int e = 0; e < 4; ++e) acc[e] += fin_prob<RMODE>(x[e], m, iz);
@@ -1329,6 +1331,7 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const void* __res
     const int t0 = tile * kFinRegTile;
     const int tb = t0 + kFinRegPos * threadIdx.x;
     const bool vec_ok = (span & 3) == 0 && tb + kFinRegPos <= span;
+    const bool vec_in = RMODE != 0 || vec_ok;  // logits, as in score_finish_kernel
     // Halo threads: [0, p) positions t0 - p + x, [p, 2p) t0 + kFinRegTile + (x - p).
     const int th = threadIdx.x < p ? t0 - p + threadIdx.x : t0 + kFinRegTile + (threadIdx.x - p);
     float best[kFinRegPos];
@@ -1352,7 +1355,7 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const void* __res
             const int r = g * W + w;
             const auto* row = logit_row<RMODE>(logits, (int64_t)job * R + r, span);
             const float m = s_m[r], iz = s_iz[r];
-            if (vec_ok) {
+            if (vec_in) {
               f32x4 x[NV];
 #pragma unroll
               for (int v = 0; v < NV; ++v) x[v] = read_logits4<RMODE>(row + tb + 4 * v);
@@ -1451,25 +1454,27 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const void* __res
   }
 }
 
-// Finish pass under the cast chain (16-bit stored logits, pool kernels 5 and
-// 7, no histogram).  A tile is 512 positions loaded, 16 bytes a lane, of which
+// Finish pass under the cast chain (16-bit stored logits, pool kernels up to
+// 9, no histogram).  A tile is 512 positions loaded, 16 bytes a lane, of which
 // the middle 496 are pooled: the neighbours are part of the tile, so there is
 // no halo path, and its stride keeps every load aligned.
 // One wave per query head (kFcHeads heads of a group at a time, the next
-// heads' first row in flight meanwhile).  With 2048-position tiles a layer of
+// heads' first rows in flight meanwhile).  With 2048-position tiles a layer of
 // a 12K prompt (28 heads over 4, float16) had 24 workgroups and took 19.4 us,
 // now 100 and 6.9; 32 heads over 8 x 131072 take 10.6 us as before, with half
-// the logits' bytes.
+// the logits' bytes.  kFcRows rows of a summed window are requested together:
+// one after the other they left 32 single heads x 40000, window 16, at 138.4 us
+// a call (135.7 with the float32 logits before), now 124.  With fewer heads
+// than waves the others take further tiles, once there are more tiles than
+// kFcGrid: 32 single heads x 40000, one row, 64.7 -> 63.0 us a call; with fewer
+// tiles the workgroups are what counts (8 x 8190: 10.4 us a call, 11.6 so).
+// Pool kernels 1, 3 and 9 in score_finish_kernel instead: 20.4 us a call for 32
+// heads over 8 x 8190, window 2, here 13.6.
 constexpr int kFcLoad = 512, kFcOut = kFcLoad - 16;
 constexpr int kFcHeads = 4;
+constexpr int kFcRows = 4;  // rows of a summed window read together
+constexpr int kFcHalf = 4;  // widest pool half-width instantiated
 constexpr int kFcGrid = 1024;
-template <int RM>
-__device__ __forceinline__ void read_logits8(const typename Logit<RM>::type* p, float (&x)[8]) {
-  typedef typename Logit<RM>::type v8 __attribute__((ext_vector_type(8)));
-  const v8 y = *reinterpret_cast<const v8*>(p);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = base2_logit<RM>((float)y[e]);
-}
 // Pooled value around strip position i (P <= 8 neighbours on either side).
 template <int POOL, int P>
 __device__ __forceinline__ float fc_pool(const float* strip, int i) {
@@ -1479,53 +1484,66 @@ __device__ __forceinline__ float fc_pool(const float* strip, int i) {
   return v;
 }
 
-template <int RM, int POOL, int P>
+// SUM: windows are summed, kFcRows rows of one read together (one row a
+// score otherwise); tp: tiles at a time, at most kFcHeads / min(G, kFcHeads).
+template <int RM, int POOL, int P, bool SUM>
 __global__ __launch_bounds__(256) void score_finish_cast_kernel(const void* __restrict__ logits,
                                                                 const float* __restrict__ stats,
                                                                 const float* __restrict__ part, int nparts, int R,
-                                                                int G, int W, int span, int sum_w, int accumulate,
+                                                                int G, int W, int span, int tp, int accumulate,
                                                                 float* __restrict__ S) {
   static_assert(RM != 0 && P <= 8, "16-bit logits, neighbours inside the tile's margin");
+  constexpr int kRows = SUM ? kFcRows : 1;
   __shared__ __align__(16) float s_a[2][kFcHeads][kFcLoad];
   __shared__ float s_m[kLogitRowsMax], s_iz[kLogitRowsMax];
-  const int wout = sum_w ? 1 : W;
+  const int wout = SUM ? 1 : W;
   const int job = blockIdx.y / wout, wo = blockIdx.y % wout;
-  const int w_lo = sum_w ? 0 : wo, w_hi = sum_w ? W : wo + 1;
+  const int w_lo = SUM ? 0 : wo, w_hi = SUM ? W : wo + 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ntiles = (span + kFcOut - 1) / kFcOut;
   constexpr float pad = POOL == 0 ? 0.f : -INFINITY;
-  // This lane's eight positions, tile * kFcOut - 8 + 8 * lane on, of one row.
-  auto row8 = [&](int tile, int g, int w, float (&x)[8]) {
-    const int t = tile * kFcOut - 8 + 8 * lane;
-    if (tile < ntiles && g < G && t >= 0 && t < span) {
-      read_logits8<RM>(logit_row<RM>(logits, (int64_t)job * R + g * W + w, span) + t, x);
-    } else {
+  typedef typename Logit<RM>::type v8 __attribute__((ext_vector_type(8)));
+  // hp heads at a time; with fewer than kFcHeads of them the other waves take
+  // further tiles: wave = (tile slot) * hp + (head slot).
+  const int hp = min(G, kFcHeads);
+  const int ts = wave / hp, hs = wave % hp;
+  const int nsteps = (ntiles + tp - 1) / tp;
+  // This lane's eight positions of the wave's tile, tile * kFcOut - 8 + 8 *
+  // lane on, of rows w .. w + kRows - 1; what is read past span is not used.
+  auto rows8 = [&](int step, int g, int w, v8 (&x)[kRows]) {
+    const int t = (step * tp + ts) * kFcOut - 8 + 8 * lane;
+    if (step < nsteps && ts < tp && g < G && t >= 0 && t < span) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = -INFINITY;
+      for (int j = 0; j < kRows; ++j)
+        if (j == 0 || w + j < w_hi)
+          x[j] = *reinterpret_cast<const v8*>(logit_row<RM>(logits, (int64_t)job * R + g * W + w + j, span) + t);
     }
   };
-  float x[8];
-  row8(blockIdx.x, wave, w_lo, x);  // in flight over the statistics
+  v8 x[kRows] = {};
+  rows8(blockIdx.x, hs, w_lo, x);  // in flight over the statistics
   finish_row_stats<false>(stats, part, nparts, job, R, s_m, s_iz);
   __syncthreads();
   const float inv_k = 1.f / (float)(2 * P + 1);
   float* o = S + ((int64_t)job * wout + wo) * span;
   int buf = 0;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int o0 = tile * kFcOut;  // first pooled position
-    const int t = o0 - 8 + 8 * lane;
+  for (int step = blockIdx.x; step < nsteps; step += gridDim.x) {
+    const int t = (step * tp + ts) * kFcOut - 8 + 8 * lane;
     float best[2] = {-INFINITY, -INFINITY};
-    for (int g0 = 0; g0 < G; g0 += kFcHeads) {
-      const int g = g0 + wave;
-      if (g < G) {
+    for (int g0 = 0; g0 < G; g0 += hp) {
+      const int g = g0 + hs;
+      if (ts < tp && g < G) {
         float acc[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-        for (int w = w_lo; w < w_hi; ++w) {
-          const int r = g * W + w;
-          if (w > w_lo) row8(tile, g, w, x);
+        for (int w = w_lo; w < w_hi; w += kRows) {
+          if (w > w_lo) rows8(step, g, w, x);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[e] += fin_prob<RM>(x[e], s_m[r], s_iz[r]);
+          for (int j = 0; j < kRows; ++j) {
+            if (w + j >= w_hi) break;
+            const float m = s_m[g * W + w + j], iz = s_iz[g * W + w + j];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] += fin_prob<RM>(base2_logit<RM>((float)x[j][e]), m, iz);
+          }
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = t + e >= 0 && t + e < span ? round_fixed<RM>(acc[e]) : pad;
@@ -1533,27 +1551,31 @@ __global__ __launch_bounds__(256) void score_finish_cast_kernel(const void* __re
         d[0] = f32x4{acc[0], acc[1], acc[2], acc[3]};
         d[1] = f32x4{acc[4], acc[5], acc[6], acc[7]};
       }
-      if (g0 + kFcHeads < G)
-        row8(tile, g + kFcHeads, w_lo, x);
+      if (g0 + hp < G)
+        rows8(step, g + hp, w_lo, x);
       else
-        row8(tile + gridDim.x, wave, w_lo, x);
+        rows8(step + gridDim.x, hs, w_lo, x);
       __syncthreads();
+      // Several tiles only with a single group of heads, so `best` serves one
+      // tile at a time.
+      for (int k = 0; k < tp; ++k) {
+        const int o0 = (step * tp + k) * kFcOut;  // first pooled position
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int i = (int)threadIdx.x + 256 * q;
-        if (i >= kFcOut) continue;
-        for (int gg = 0; gg < kFcHeads && g0 + gg < G; ++gg) {
-          float v = fc_pool<POOL, P>(s_a[buf][gg], 8 + i);
-          if constexpr (POOL == 0) v *= inv_k;
-          best[q] = fmaxf(best[q], round_fixed<RM>(v));
+        for (int q = 0; q < 2; ++q) {
+          const int i = (int)threadIdx.x + 256 * q;
+          if (i >= kFcOut || o0 + i >= span) continue;
+          for (int gg = 0; gg < hp && g0 + gg < G; ++gg) {
+            float v = fc_pool<POOL, P>(s_a[buf][k * hp + gg], 8 + i);
+            if constexpr (POOL == 0) v *= inv_k;
+            best[q] = fmaxf(best[q], round_fixed<RM>(v));
+          }
+          if (g0 + hp >= G) {
+            o[o0 + i] = accumulate ? o[o0 + i] + best[q] : best[q];
+            best[q] = -INFINITY;
+          }
         }
       }
       buf ^= 1;  // the next strips: this buffer may still be read
-    }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int i = (int)threadIdx.x + 256 * q;
-      if (i < kFcOut && o0 + i < span) o[o0 + i] = accumulate ? o[o0 + i] + best[q] : best[q];
     }
   }
 }
@@ -2162,32 +2184,50 @@ static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* 
   }
   const float* fpart = fold_in_finish ? part : nullptr;
   const int acc_out = (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, sum_out = (a.flags & HC_SCORE_SUM_WINDOW) ? 1 : 0;
-  if (via_logits && rm != 0 && pool57 && !hist) {
+  if (via_logits && rm != 0 && kernel <= 2 * kFcHalf + 1 && !hist) {
     if (a.span > 0) {
       const int ntiles = (a.span + kFcOut - 1) / kFcOut;
-      // Several tiles a workgroup where there are more than kFcGrid of them:
-      // each folds the row statistics once.
-      const int64_t per = cast_window ? 1 : ((int64_t)ntiles * njobs * wout + kFcGrid - 1) / kFcGrid;
-      const dim3 cgrid((unsigned)((ntiles + per - 1) / per), njobs * wout);
-#define HC_FCAST(RM, PL, P)                                                                                        \
-  do {                                                                                                            \
-    if (cast_window)                                                                                              \
-      hipLaunchKernelGGL((score_finish_window_kernel<RM, PL, P>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts, \
-                         a.R, a.G, a.W, a.span, acc_out, scores);                                                 \
-    else                                                                                                          \
-      hipLaunchKernelGGL((score_finish_cast_kernel<RM, PL, P>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts,   \
-                         a.R, a.G, a.W, a.span, sum_out, acc_out, scores);                                        \
-  } while (0)
-#define HC_FCAST_P(RM, PL)       \
-  do {                           \
-    if (kernel == 5)             \
-      HC_FCAST(RM, PL, 2);       \
-    else                         \
-      HC_FCAST(RM, PL, 3);       \
+      // Several tiles at a time, and several steps a workgroup, where there are
+      // more than kFcGrid of them: each folds the row statistics once.
+      const int tp = cast_window || (int64_t)ntiles * njobs * wout <= kFcGrid ? 1 : kFcHeads / std::min(a.G, kFcHeads);
+      const int nsteps = (ntiles + tp - 1) / tp;
+      const int64_t per = cast_window ? 1 : ((int64_t)nsteps * njobs * wout + kFcGrid - 1) / kFcGrid;
+      const dim3 cgrid((unsigned)((nsteps + per - 1) / per), njobs * wout);
+#define HC_FCAST(RM, PL, P, SUM)                                                                                  \
+  hipLaunchKernelGGL((score_finish_cast_kernel<RM, PL, P, SUM>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts, \
+                     a.R, a.G, a.W, a.span, tp, acc_out, scores)
+#define HC_FCAST_SUM(RM, PL, P)         \
+  case P:                               \
+    if (sum_out && a.W > 1)             \
+      HC_FCAST(RM, PL, P, true);        \
+    else                                \
+      HC_FCAST(RM, PL, P, false);       \
+    break
+#define HC_FWINDOW(RM, PL, P)                                                                                     \
+  hipLaunchKernelGGL((score_finish_window_kernel<RM, PL, P>), cgrid, dim3(256), 0, s, A, stats, fpart, nparts,    \
+                     a.R, a.G, a.W, a.span, acc_out, scores)
+#define HC_FCAST_P(RM, PL)                          \
+  do {                                              \
+    if (cast_window) {                              \
+      if (kernel == 5)                              \
+        HC_FWINDOW(RM, PL, 2);                      \
+      else                                          \
+        HC_FWINDOW(RM, PL, 3);                      \
+    } else {                                        \
+      switch (kernel / 2) {                         \
+        HC_FCAST_SUM(RM, PL, 0);                        \
+        HC_FCAST_SUM(RM, PL, 1);                        \
+        HC_FCAST_SUM(RM, PL, 2);                        \
+        HC_FCAST_SUM(RM, PL, 3);                        \
+        HC_FCAST_SUM(RM, PL, 4);                        \
+      }                                             \
+    }                                               \
   } while (0)
       if (rm == 1) { if (pooling == 0) HC_FCAST_P(1, 0); else HC_FCAST_P(1, 1); }
       else { if (pooling == 0) HC_FCAST_P(2, 0); else HC_FCAST_P(2, 1); }
 #undef HC_FCAST_P
+#undef HC_FWINDOW
+#undef HC_FCAST_SUM
 #undef HC_FCAST
       if ((rc = check_launch("hc_score(finish)"))) return rc;
     }

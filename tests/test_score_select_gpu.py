@@ -97,8 +97,11 @@ def test_bf16_cast_chain(dev):
     (1, 32, 17000, True),  # more partials than a tile's logits: the merge launch
     # fewer than 32 rows: one wave per query head, four heads at a time
     (1, 1, 1, False), (4, 1, 496, False), (5, 1, 497, False), (7, 1, 1489, False), (9, 1, 505, False),
-    (3, 4, 1000, False), (2, 8, 991, True), (1, 16, 513, True)])
-@pytest.mark.parametrize("pooling,kernel", [("avgpool", 5), ("maxpool", 7)])
+    (3, 4, 1000, False), (2, 8, 991, True), (1, 16, 513, True),
+    (2, 2, 1026, False), (1, 8, 1031, True), (3, 8, 2051, False)])
+# Kernels up to 9 have instances of their own over fewer than 32 rows, 11 none.
+@pytest.mark.parametrize("pooling,kernel", [("avgpool", 5), ("maxpool", 7), ("avgpool", 1), ("avgpool", 3),
+                                            ("maxpool", 9), ("avgpool", 11)])
 def test_cast_chain_16bit_logits(dev, dt, G, W, L, keep, pooling, kernel):
     """Scores under the cast chain, whose logits are stored in 16 bits, over
     tile edges, window sizes and group sizes.  A 32-bit sum on the other side
@@ -119,6 +122,23 @@ def test_cast_chain_16bit_logits(dev, dt, G, W, L, keep, pooling, kernel):
     assert (s == ref).mean() >= 0.9
 
 
+@pytest.mark.parametrize("G,W", [(1, 1), (1, 4), (2, 1), (2, 8), (3, 1)])
+def test_cast_chain_several_tiles_at_a_time(dev, G, W):
+    """Enough tiles (over 1024) that the waves of a workgroup share out tiles
+    as well as query heads, at tails of one to three tiles, against the oracle
+    (tolerance as test_cast_chain_16bit_logits) and the same jobs scored alone."""
+    jobs, L = 420, 1000 + 8 * G + W
+    q, k = qk(dev, 1, jobs * G, jobs, W, L, torch.bfloat16, 3 * G + W)
+    s = compress.window_scores(q, k, range(jobs), G, W, "avgpool", 5, round_dtype=torch.bfloat16)
+    for j in (0, 211, jobs - 1):
+        alone = compress.window_scores(q, k, [j], G, W, "avgpool", 5, round_dtype=torch.bfloat16)
+        ref = O.window_scores(as_np(q)[0, j * G:(j + 1) * G][None], as_np(k)[0, j:j + 1], "avgpool", 5,
+                              window_keep=False, io_dtype="bfloat16")[0]
+        got = as_np(s[j])
+        assert (np.abs(got - ref) <= 2 * 2.0 ** -7 * np.abs(ref)).all()
+        assert np.mean(got == as_np(alone[0])) > 0.99
+
+
 @pytest.mark.parametrize("G,W,L", [(1, 1, 1), (1, 1, 7), (2, 1, 33), (4, 1, 1001), (1, 8, 1030), (7, 2, 1023), (2, 4, 515)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_few_rows_uncast_odd_spans(dev, G, W, L, dtype):
@@ -131,6 +151,29 @@ def test_few_rows_uncast_odd_spans(dev, G, W, L, dtype):
     ref = O.window_scores(np.stack([qn[0, h * G:(h + 1) * G, -W:] for h in range(Hkv)]), kn[0], "avgpool", 5,
                           window_keep=False)
     assert rel_err(as_np(s), ref) < 2e-4
+
+
+@pytest.mark.parametrize("L", [1025, 2051, 4098])
+@pytest.mark.parametrize("kernel", [3, 5])
+def test_cast_scores_with_histograms_at_odd_spans(dev, L, kernel):
+    """The passes that also build the first-digit histograms, over 16-bit
+    logits of odd spans: the scores of the passes without, and the counts of
+    their leading key bits."""
+    G, S = 4, 5
+    g = torch.Generator().manual_seed(L)
+    steps = torch.randn(1, 2 * G, S, 128, generator=g).bfloat16().to(dev)
+    k = torch.randn(1, 2, L, 128, generator=g).bfloat16().to(dev)
+    store = KVStore([L + 8] * 2, torch.bfloat16, dev)
+    store.write_rows(k, k, [(0, 0), (0, 1)], [0, 1], [L, L])
+    hist = torch.full((2 * S, ops.HIST_BINS), 7, dtype=torch.int32, device=dev)
+    got = compress.pivot_step_scores(steps, store, [0, 1], [0, 1], G, L, "avgpool", kernel, round_dtype=torch.bfloat16,
+                                     hist=hist)
+    plain = compress.pivot_step_scores(steps, store, [0, 1], [0, 1], G, L, "avgpool", kernel,
+                                       round_dtype=torch.bfloat16)
+    assert torch.equal(got, plain)
+    bits = (as_np(got).reshape(2 * S, L).astype(np.float32).view(np.uint32) | np.uint32(1 << 31)) >> 20
+    ref = np.stack([np.bincount(r, minlength=ops.HIST_BINS) for r in bits.astype(np.int64)])
+    assert np.array_equal(as_np(hist).astype(np.int64), ref)
 
 
 @pytest.mark.parametrize("W,L,jobs,stored", [
