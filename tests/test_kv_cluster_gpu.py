@@ -103,9 +103,8 @@ def test_pyramidkv_cluster(dev, layer):
 
 
 def test_h2o_cluster(dev):
-    """530 float32 query rows: four 128-row scorer calls (probability pass),
-    then 16- and 2-row ones (logit-store pass), accumulated into one score
-    row."""
+    """Scores of 530 float32 query rows against the oracle's, and the kept
+    rows of update_kv."""
     B, H, L, G = 1, 4, 530, 2
     print("h2o", flush=True)
     q, k, v = _inputs(dev, B, H, L, 50)

@@ -208,6 +208,28 @@ def test_cast_window_workspace(dev, W, L, jobs, stored):
         assert (s == ref).mean() >= 0.9
 
 
+@pytest.mark.parametrize("G,W,kernel,rounded", [
+    (4, 1, 5, None), (4, 1, 9, None),                       # stored float32 logits
+    (1, 32, 5, None), (8, 8, 5, None), (1, 32, 31, None),   # two passes over the keys
+    (4, 1, 5, torch.bfloat16), (2, 4, 3, torch.bfloat16),   # stored 16-bit logits: a few rows,
+    (4, 1, 11, torch.bfloat16),                             # a wide pool kernel,
+    (1, 32, 5, torch.bfloat16), (2, 32, 7, torch.bfloat16)])  # summed windows
+@pytest.mark.parametrize("L", [1100, 1101])
+def test_accumulated_scores(dev, G, W, kernel, rounded, L):
+    """HC_SCORE_ACCUMULATE adds the call's scores to what the output holds, in
+    float32, on every route."""
+    Hkv = 2
+    q, k = qk(dev, 1, Hkv * G, Hkv, W, L, torch.bfloat16, L + G + W + kernel)
+    flags = _lib.HC_SCORE_SUM_WINDOW | _lib.HC_SCORE_CAUSAL_WINDOW | compress.ROUND_FLAGS[rounded]
+    off_q, off_k = (torch.arange(Hkv, device=dev) * h for h in (G * q.stride(1), k.stride(1)))
+
+    def score(more=0, out=None):
+        return ops.score(q, off_q, q.stride(1), q.stride(2), k, off_k, k.stride(2), L, G, W, L - W, "avgpool", kernel,
+                         1 / math.sqrt(128), flags=flags | more, out=out)
+    base = torch.rand((Hkv, 1, L - W), device=dev)
+    assert torch.equal(score(_lib.HC_SCORE_ACCUMULATE, base.clone()), base + score())
+
+
 def test_pivot_step_scores_read_store_in_place(dev):
     B, Hq, Hkv, L, S, G = 1, 32, 8, 2500, 5, 4
     q, k = qk(dev, B, Hq, Hkv, 1, L, torch.bfloat16, 5, strided=False)
