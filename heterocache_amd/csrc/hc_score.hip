@@ -2125,6 +2125,24 @@ static int launch_probs_pool(ScoreArgs a, int njobs, int pooling, int kernel, St
   return HC_OK;
 }
 
+// The finish from stored logits that score_finish_cast_kernel and
+// score_finish_window_kernel do not serve.
+template <int RM, int POOL, bool HIST>
+static void launch_finish(const ScoreArgs& a, dim3 grid, const float* logits, const float* stats, const float* part,
+                          int nparts, int sum_w, int kernel, int accumulate, float* scores, uint32_t* hist,
+                          hipStream_t s) {
+  if constexpr (RM == 0 || HIST) {
+    if (kernel == 5 || kernel == 7) {
+      auto fn = kernel == 5 ? score_finish_reg_kernel<RM, POOL, HIST, 2> : score_finish_reg_kernel<RM, POOL, HIST, 3>;
+      hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, logits, stats, part, nparts, a.R, a.G, a.W, a.span, sum_w, kernel,
+                         accumulate, scores, hist);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((score_finish_kernel<RM, POOL, HIST>), grid, dim3(256), 0, s, logits, stats, part, nparts, a.R,
+                     a.G, a.W, a.span, sum_w, kernel, accumulate, scores, hist);
+}
+
 template <typename T, bool STORE>
 static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* scores, void* ws, size_t ws_bytes,
                         uint32_t* hist, hipStream_t s) {
@@ -2235,43 +2253,20 @@ static int launch_score(ScoreArgs a, int njobs, int pooling, int kernel, float* 
   }
   if (via_logits) {
     if (a.span > 0) {
-      const bool reg_pool = pool57;
-      const int ntiles = (a.span + (reg_pool ? kFinRegTile : kFinTile) - 1) / (reg_pool ? kFinRegTile : kFinTile);
-      const int rows = njobs * wout;
-      const int ht = reg_pool ? kFinRegHistTiles : kFinHistTiles;
-      const int per_row = hist ? (ntiles + ht - 1) / ht : ntiles;
-      const dim3 fgrid(per_row, rows);
-      const int sum_w = sum_out;
-      const int rmode = rm;
-#define HC_FINISH2(RM, PL, HI)                                                                              \
-  do {                                                                                                      \
-    if (kernel == 5 && (RM == 0 || HI))                                                                     \
-      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, (RM != 0 || HI), 2>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
-                         nparts, a.R,                                                                 \
-                         a.G, a.W, a.span, sum_w, kernel, (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, scores,    \
-                         hist);                                                                             \
-    else if (kernel == 7 && (RM == 0 || HI))                                                                \
-      hipLaunchKernelGGL((score_finish_reg_kernel<RM, PL, (RM != 0 || HI), 3>), fgrid, dim3(256), 0, s, A, stats, fpart,   \
-                         nparts, a.R,                                                                 \
-                         a.G, a.W, a.span, sum_w, kernel, (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, scores,    \
-                         hist);                                                                             \
-    else                                                                                                    \
-      hipLaunchKernelGGL((score_finish_kernel<RM, PL, HI>), fgrid, dim3(256), 0, s, A, stats, fpart, nparts,  \
-                         a.R, a.G, a.W,                                                               \
-                         a.span, sum_w, kernel, (a.flags & HC_SCORE_ACCUMULATE) ? 1 : 0, scores, hist);      \
+      const int ntiles = (a.span + (pool57 ? kFinRegTile : kFinTile) - 1) / (pool57 ? kFinRegTile : kFinTile);
+      const int ht = pool57 ? kFinRegHistTiles : kFinHistTiles;
+      const dim3 fgrid(hist ? (ntiles + ht - 1) / ht : ntiles, njobs * wout);
+#define HC_FINISH(RM, PL)                                                                                     \
+  do {                                                                                                        \
+    if (hist)                                                                                                 \
+      launch_finish<RM, PL, true>(a, fgrid, A, stats, fpart, nparts, sum_out, kernel, acc_out, scores, hist, s);  \
+    else                                                                                                      \
+      launch_finish<RM, PL, false>(a, fgrid, A, stats, fpart, nparts, sum_out, kernel, acc_out, scores, hist, s); \
   } while (0)
-#define HC_FINISH(RM, PL)          \
-  do {                             \
-    if (hist)                      \
-      HC_FINISH2(RM, PL, true);    \
-    else                           \
-      HC_FINISH2(RM, PL, false);   \
-  } while (0)
-      if (rmode == 0) { if (pooling == 0) HC_FINISH(0, 0); else HC_FINISH(0, 1); }
-      else if (rmode == 1) { if (pooling == 0) HC_FINISH(1, 0); else HC_FINISH(1, 1); }
+      if (rm == 0) { if (pooling == 0) HC_FINISH(0, 0); else HC_FINISH(0, 1); }
+      else if (rm == 1) { if (pooling == 0) HC_FINISH(1, 0); else HC_FINISH(1, 1); }
       else { if (pooling == 0) HC_FINISH(2, 0); else HC_FINISH(2, 1); }
 #undef HC_FINISH
-#undef HC_FINISH2
       if ((rc = check_launch("hc_score(finish)"))) return rc;
     }
     return HC_OK;
