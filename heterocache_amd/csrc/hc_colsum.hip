@@ -17,12 +17,14 @@
 // the accumulators; nothing of size L x L leaves the registers.
 //
 // What bounds it: per 16 x 16 block 64 matrix cycles, and 4 elements a lane
-// of fma + v_exp (8 cycles) + add, which the other waves of the SIMD (four
-// resident at 123 registers) run beside the matrix instructions, and under
-// load the chip's power: the first launches after idle take 0.54 ms a pass at
-// 32 heads x 8190 tokens, sustained ones 0.51-0.70 with the clock.  (So an
-// order with one block's exponentials between the next block's matrix
-// instructions, three waves a SIMD, measured no faster: 1.11 ms against 1.07.)
+// of fma + v_exp (a quarter of the VALU rate) + add, which the other waves of
+// the SIMD (four resident at 124 and 126 registers) run beside the matrix
+// instructions, and under load the chip's power.  At 32 heads x 8190 tokens
+// the matrix pipe is busy half of the cycles, waves wait for dependencies half
+// of theirs, LDS is active in 12 and 16 % without conflicts, and a pass takes
+// 0.54-0.67 ms with the clock.  (So an order with one block's exponentials
+// between the next block's matrix instructions, three waves a SIMD, measured
+// no faster: 1.11 ms against 1.07.)
 // Pass 1 takes no maximum in its loop: the row reference m is the maximum of
 // the first rows, and an iteration's sums are only redone against a new
 // maximum when they pass kCsLazy (the sums are needed anyway; one compare

@@ -35,7 +35,7 @@
 //    only when a tile's probability sums, which are formed anyway, exceed
 //    kPfLazy.  Without the 32 maxima a lane and their cross-lane folds per 64
 //    keys: 15.41 -> 14.66 ms for 8192 queries over 131072 keys (32 heads over
-//    8, bf16; 1105 -> 1162 TFLOP/s), 0.53 -> 0.50 ms for 8003 over 8003.
+//    8, bf16; 1105 -> 1162 TFLOP/s), 0.49 -> 0.47 ms for 8003 over 8003.
 //    (48 or 64 queries a wave, so that an LDS read feeds 3 or 4 MFMAs, leave
 //    two waves or one per SIMD: 15.9 and 19.5 ms.)
 #include <algorithm>

@@ -30,7 +30,8 @@
 //     max over g -> S[job][w'][t].
 //  3b. (stored logits) score_finish_kernel: the same from the stored logits
 //     (for pool kernels 5 and 7 score_finish_reg_kernel: pooling in
-//     registers; under the cast chain score_finish_cast_kernel and
+//     registers; under the cast chain, without histograms,
+//     score_finish_cast_kernel for pool kernels up to 9 and
 //     score_finish_window_kernel).
 // CAKE scoring (hc_cake_score) runs phases 1-2, the probability pass with
 // window moments, and its own pooling and reductions.
@@ -1582,10 +1583,10 @@ __global__ __launch_bounds__(256) void score_finish_cast_kernel(const void* __re
 
 // The same for summed windows of whole 16-row tiles (R <= kCastLogitRows):
 // wave rg sums rows 16n + 4rg + [0, 4) of a head's window, and the four
-// waves' sums are added in score_probs_pool_kernel's order, so the scores are
-// the ones that pass forms.  Its second read of the keys (256 bytes a token
-// and job) and their products are replaced by the logits' write and read
-// (2R bytes each).
+// waves' sums are added in score_probs_pool_kernel's order (the row statistics
+// in another: 256 / R partial folds a row).  That pass's second read of the
+// keys (256 bytes a token and job) and their products are replaced by the
+// logits' write and read (2R bytes each).
 // Measured, per call, against two passes over the keys (us): 32 rows, 32 jobs
 // x 700 keys 18.0 -> 16.6, x 8192 39.7 -> 26.6, x 65536 206 -> 162, x 131072
 // (256 MiB of logits) 391 -> 310, 64 jobs x 65536 391 -> 304; 64 rows, 32 jobs
