@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kScoreWaves * 64) void score_stats_kernel(ScoreArgs
 // of its token.  A transpose over the groups then gives a lane eight
 // consecutive tokens, so that the logits, in score_stats_kernel's form
 // ([job][R][span], see Logit), leave as 16-byte units (single stores and
-// float32 throughout: 58.3 us for eight heads x 128K, four rows; 53.9 with
+// float32 throughout: 58.3 us for eight heads x 128K, four rows; 52.2 with
 // 16-bit units); every workgroup writes one
 // (max, sum) partial per row, so the merge and finish passes are shared.
 // NR: rows held per lane (R rounded up to 4, 8 or 16).
@@ -1462,7 +1462,7 @@ __global__ __launch_bounds__(256) void score_finish_reg_kernel(const void* __res
 // One wave per query head (kFcHeads heads of a group at a time, the next
 // heads' first rows in flight meanwhile).  With 2048-position tiles a layer of
 // a 12K prompt (28 heads over 4, float16) had 24 workgroups and took 19.4 us,
-// now 100 and 6.9; 32 heads over 8 x 131072 take 10.6 us as before, with half
+// now 100 and 6.8; 32 heads over 8 x 131072 take 10.4 us as before (10.6), with half
 // the logits' bytes.  kFcRows rows of a summed window are requested together:
 // one after the other they left 32 single heads x 40000, window 16, at 138.4 us
 // a call (135.7 with the float32 logits before), now 124.  With fewer heads
