@@ -781,14 +781,18 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(const PfAr
   }
 }
 
-// Slices of 16 channels while their workgroups are all resident at once;
-// with more queries (short chunks) the device is full anyway, and one
-// workgroup per query reads each (m, l) once.
+// Slices of 16 channels while their workgroups are all resident at once (with
+// more queries, short chunks, the device is full anyway) and the splits take a
+// workgroup of a whole query more than two rounds of loads, 16 splits each.
+// One query per head, us a call, whole against sliced, KV heads x splits: 8 x 1
+// 11.8 / 12.3, 4 x 15 12.7 / 13.7, 8 x 31 18.4 / 18.5, 16 x 32 44.9 / 45.2, 8 x
+// 39 24.7 / 23.9, 4 x 78 26.9 / 24.5, 8 x 64 50.7 / 49.0, 4 x 128 44.2 / 39.5.
 constexpr int64_t kMergeSlicedGrid = 2048;
+constexpr int kMergeWholeSplits = 32;
 template <typename T>
 int launch_merge(const PfArgs& a, hipStream_t stream) {
   const int64_t nq = (int64_t)(a.rows / a.Hkv) * a.Hq * a.Lq;
-  if (nq * (HC_HEAD_DIM / 16) <= kMergeSlicedGrid)
+  if (a.nsplit > kMergeWholeSplits && nq * (HC_HEAD_DIM / 16) <= kMergeSlicedGrid)
     hipLaunchKernelGGL((prefill_merge_kernel<T, 16>), dim3((unsigned)nq, HC_HEAD_DIM / 16), dim3(kMergeThreads), 0,
                        stream, a);
   else

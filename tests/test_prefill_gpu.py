@@ -271,6 +271,8 @@ DECODE_SHAPED_CASES = [
     (1, 8, 8, 16, 3001),      # no GQA, 16 queries, a ragged last tile
     (3, 4, 2, 8, 1100),       # GQA 2 x 8 queries, batch 3
     (4, 32, 32, 16, 1030),    # more queries than the sliced merge takes
+    (1, 2, 1, 1, 16384),      # 32 splits: whole queries are merged
+    (1, 2, 1, 2, 16900),      # 33: sliced by 16 channels
     (1, 4, 1, 1, 4129),       # one KV row, a tile of one key
 ]
 
